@@ -445,6 +445,19 @@ emu_v4f emu_mfma_f32_16x16x32_f16(emu_v8h a, emu_v8h b, emu_v4f c) {
   return d;
 }
 
+emu_v4f emu_mfma_f32_16x16x4f32(float a, float b, emu_v4f c) {
+  struct P {
+    float a, b;
+  } mine{a, b};
+  const unsigned char* s = emu::wave_exchange(&mine, sizeof(P), emu::kOpMfma);
+  const int l = emu::cur()->lane, n = l & 15, g = l >> 4;
+  emu_v4f d = c;
+  for (int r = 0; r < 4; ++r)
+    for (int k = 0; k < 4; ++k)
+      d[r] = std::fmaf(emu::lane_value<P>(s, 4 * g + r + 16 * k).a, emu::lane_value<P>(s, n + 16 * k).b, d[r]);
+  return d;
+}
+
 // ---- runtime API ------------------------------------------------------------------------
 namespace {
 std::map<void*, size_t>& allocs() {

@@ -241,6 +241,8 @@ typedef _Float16 emu_v8h __attribute__((ext_vector_type(8)));
 // of lane l is D[4 * (l / 16) + r][l % 16].
 emu_v4i emu_mfma_i32_16x16x64_i8(emu_v4i a, emu_v4i b, emu_v4i c);
 emu_v4f emu_mfma_f32_16x16x32_f16(emu_v8h a, emu_v8h b, emu_v4f c);
+// (K = 4, one value per lane: k = l / 16; four fused steps in ascending k)
+emu_v4f emu_mfma_f32_16x16x4f32(float a, float b, emu_v4f c);
 inline emu_v4i emu_mfma_i8_6(emu_v4i a, emu_v4i b, emu_v4i c, int, int, int) {
   return emu_mfma_i32_16x16x64_i8(a, b, c);
 }
@@ -249,6 +251,8 @@ inline emu_v4f emu_mfma_f16_6(emu_v8h a, emu_v8h b, emu_v4f c, int, int, int) {
 }
 #define __builtin_amdgcn_mfma_i32_16x16x64_i8(...) emu_mfma_i8_6(__VA_ARGS__)
 #define __builtin_amdgcn_mfma_f32_16x16x32_f16(...) emu_mfma_f16_6(__VA_ARGS__)
+inline emu_v4f emu_mfma_f32_6(float a, float b, emu_v4f c, int, int, int) { return emu_mfma_f32_16x16x4f32(a, b, c); }
+#define __builtin_amdgcn_mfma_f32_16x16x4f32(...) emu_mfma_f32_6(__VA_ARGS__)
 
 // ---- runtime API ---------------------------------------------------------------------
 hipError_t hipGetDeviceCount(int* n);

@@ -58,3 +58,29 @@ def test_qgemm_f16_declines_non_codebook_and_pairs(dev):
     finally:
         L.ifr_linear_free(dev.ctx, d1)
         L.ifr_linear_free(dev.ctx, d2)
+
+
+@pytest.mark.parametrize("bits,N,K,M,shift", [(2, 16, 128, 2, 0), (4, 80, 256, 17, 0), (2, 1024, 128, 361, 0),
+                                              (4, 1024, 128, 800, 0), (8, 1024, 128, 801, 0), (2, 144, 256, 33, 2),
+                                              (4, 48, 128, 1, 2)])
+def test_qgemm_f16_row_blocks_and_unaligned_rows(dev, bits, N, K, M, shift):
+    """Each row-block size the launch picks (16, 32 and 64 rows), partial last
+    blocks and column tiles, and activations that start off a 16-byte
+    boundary, bit for bit against the oracle."""
+    rng = np.random.default_rng(bits * 11 + M)
+    lin = ia.make_linear(N, K, bits, rng)
+    dl = C.c_void_p()
+    ia.check(L.ifr_linear_upload(dev.ctx, C.byref(lin.struct), C.byref(dl)), "upload")
+    a = (rng.standard_normal((M, K)) * 2).astype(np.float16)
+    ad = dev.upload(np.concatenate([np.zeros(shift // 2, np.uint16), a.view(np.uint16).reshape(-1)]))
+    od = dev.alloc(M * N * 2)
+    try:
+        announce(f"fp16 GEMM bits={bits} N={N} K={K} M={M} shift={shift}")
+        ia.check(L.ifr_quant_gemm_f16(dev.ctx, dl, C.c_void_p(ad.p.value + shift), M, C.c_float(0.37), od.p), "f16 gemm")
+        ref = np.empty((M, N), np.uint16)
+        po.oracle().or_qgemm_f16(ptr(a.view(np.uint16)), M, C.byref(lin.struct), np.float32(0.37), ptr(ref))
+        assert np.array_equal(dev.download(od, np.uint16, (M, N)), ref)
+    finally:
+        ad.free()
+        od.free()
+        L.ifr_linear_free(dev.ctx, dl)
