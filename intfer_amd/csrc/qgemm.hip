@@ -100,9 +100,25 @@ namespace {
 // int8 B operand: operand dword d holds codes j = 4d..4d+3 in bytes 0..3
 // (INT2: byte b of dword d is bits [8b + 2d, +2) of the packed dword; INT4:
 // bits [8b + 4(d%2), +4) of packed dword d/2; INT8: stored directly).
-template <int BITS>
+template <int BITS, bool NT = true>
 __device__ __forceinline__ void load_raw(const uint32_t* __restrict__ base, int lane,
                                          uint32_t (&w)[BITS / 2]) {
+  if constexpr (!NT) {  // codes that other workgroups read again from the L2
+    if constexpr (BITS == 2) {
+      w[0] = base[lane];
+    } else if constexpr (BITS == 4) {
+      const uint2 x = reinterpret_cast<const uint2*>(base)[lane];
+      w[0] = x.x;
+      w[1] = x.y;
+    } else {
+      const uint4 x = reinterpret_cast<const uint4*>(base)[lane];
+      w[0] = x.x;
+      w[1] = x.y;
+      w[2] = x.z;
+      w[3] = x.w;
+    }
+    return;
+  }
   if constexpr (BITS == 2) {
     w[0] = __builtin_nontemporal_load(base + lane);
   } else if constexpr (BITS == 4) {
@@ -850,6 +866,155 @@ __global__ __launch_bounds__(256) void qgemm_full(KParams p) {
   store_tiles<WM, WN, EPI, DUMP>(p, lds_f, acc, asr, row0, tile0, wave, lane);
 }
 
+// ---- large M: bound by instruction issue, the fold's fp32 operations and the
+// MFMAs not overlapping on a SIMD (a register-only loop of this body: 197 ns for
+// 64 x 32 outputs a group, 240 with 32-row waves, whose codes are unpacked twice
+// as often; the MFMAs alone 125), and by the operand traffic beside it.  So a
+// wave takes 64 rows, the codes unpacked once for four row tiles; A of the next
+// group is staged in LDS for the 4 waves (64 rows x 16 WN columns each, side by
+// side) through registers, two buffers and one barrier a group, so the vector
+// memory unit moves each A byte once per workgroup; a wave's codes and scale |
+// zero pairs of two groups are in flight in registers, each slot refilled as
+// soon as its column tile is unpacked, with plain loads (the other row blocks
+// read them from the L2: streaming loads 577, plain 530 us).  Same fold, same
+// group order, same bits.  Against qgemm_rows at M = 2160 (INT2): gate/up
+// 5120 -> 2 x 17408 642 -> 530 us, down 17408 -> 5120 455 -> 300, QKV 146 -> 116,
+// O 108 -> 95; INT4 at M = 1024: gate/up 436 -> 307, down 275 -> 170.
+template <int BITS, int WM, int WN, int EPI, bool FF>
+__global__ __launch_bounds__(256, 2) void qgemm_tall(KParams p) {
+  constexpr int BM = 16 * WM, BN = 64 * WN, SP = BM + 4;
+  constexpr int NA = WM / 2;  // 1 KB A tiles of a group per wave: 2 WM over 4 waves
+  static_assert(WM % 2 == 0, "the waves share the A copies evenly");
+  extern __shared__ v4f lds_f4[];
+  float* const lds_f = reinterpret_cast<float*>(lds_f4);
+  int8_t* const A_l = reinterpret_cast<int8_t*>(lds_f4);              // [2][2 WM][1 KB]
+  float* const S_l = reinterpret_cast<float*>(A_l + 2 * 2 * WM * 1024);  // [ng][SP]
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lrow = lane & 15, lgrp = lane >> 4;
+  const int ntiles = p.N >> 4, ng = p.ng;
+  int bx = blockIdx.x, by = blockIdx.y;
+  if (p.swz > 0) {  // the column order of qgemm_rows
+    const int x = blockIdx.x & 7, local = blockIdx.x >> 3, per = (p.nbx + 7) >> 3;
+    const int G = min(p.swz, per);
+    const int gi = local / (G * p.nby), r = local - gi * G * p.nby;
+    const int Gg = min(G, per - gi * G);
+    by = r / Gg;
+    bx = x + 8 * (gi * G + (r - by * Gg));
+    if (bx >= p.nbx || by >= p.nby) return;  // padding (before any barrier)
+  }
+  const int bm0 = by * BM, tile0 = bx * (BN / 16) + WN * wave;
+
+  // A: chunk ch = 2 rt + h is row tile rt's K step h of the group (row tiles
+  // past the last one read the last, whose outputs are never stored)
+  uint32_t asrc[NA];  // 1 KB tiles; wave-uniform, so the loads take a scalar base
+#pragma unroll
+  for (int q = 0; q < NA; ++q) {
+    const int ch = wave * NA + q;
+    asrc[q] = (uint32_t)(min((bm0 >> 4) + (ch >> 1), (p.M - 1) >> 4) * p.nsteps + (ch & 1));
+  }
+  v4i st[NA];
+  auto load_a = [&](int g) {
+#pragma unroll
+    for (int q = 0; q < NA; ++q) st[q] = reinterpret_cast<const v4i*>(p.a + (size_t)(asrc[q] + 2 * g) * 1024)[lane];
+  };
+  auto store_a = [&](int g) {
+#pragma unroll
+    for (int q = 0; q < NA; ++q)
+      *reinterpret_cast<v4i*>(A_l + ((g & 1) * 2 * WM + wave * NA + q) * 1024 + 16 * lane) = st[q];
+  };
+  int tl[WN];
+#pragma unroll
+  for (int j = 0; j < WN; ++j) tl[j] = min(tile0 + j, ntiles - 1);
+  struct Slot {
+    uint32_t B[2][WN][BITS / 2];
+    uint32_t z[WN];
+  } ring[2];
+  auto fetch = [&](Slot& o, int j, int g) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+      load_raw<BITS, false>(p.codes + ((size_t)tl[j] * p.nsteps + 2 * g + h) * 64 * (BITS / 2), lane, o.B[h][j]);
+    o.z[j] = (p.sz + ((size_t)tl[j] * ng + g) * 16)[lrow];
+  };
+  load_a(0);
+#pragma unroll
+  for (int j = 0; j < WN; ++j) fetch(ring[0], j, 0);
+#pragma unroll
+  for (int j = 0; j < WN; ++j) fetch(ring[1], j, min(1, ng - 1));
+  // S (FF: Y = 1.5 * 2^23 + C * S) of the block's rows, [group][row]; each
+  // wave reads whole rows.  Rows past M read row M - 1.
+  {
+    constexpr float C = (float)((1 << BITS) - 1);
+    for (int r = wave; r < BM; r += 4)
+      for (int g = lane; g < ng; g += 64) {
+        const float sv = p.gs[(size_t)min(bm0 + r, p.M - 1) * ng + g];
+        S_l[g * SP + r] = FF ? kFoldBiasF + C * sv : sv;
+      }
+  }
+  store_a(0);
+  load_a(min(1, ng - 1));
+  v4f acc[WM][WN];
+#pragma unroll
+  for (int i = 0; i < WM; ++i)
+#pragma unroll
+    for (int j = 0; j < WN; ++j) acc[i][j] = (v4f){0.f, 0.f, 0.f, 0.f};
+  __syncthreads();
+
+  auto group = [&](int g, Slot& o) {
+    const int8_t* Ag = A_l + (g & 1) * 2 * WM * 1024 + 16 * lane;
+    v4i A[2][WM];
+    v4f S[WM];
+#pragma unroll
+    for (int i = 0; i < WM; ++i) {
+#pragma unroll
+      for (int h = 0; h < 2; ++h) A[h][i] = *reinterpret_cast<const v4i*>(Ag + (2 * i + h) * 1024);
+      S[i] = *reinterpret_cast<const v4f*>(&S_l[g * SP + 16 * i + 4 * lgrp]);
+    }
+    // the other buffer's readers passed the barrier of group g - 1
+    store_a(g + 1);
+    load_a(min(g + 2, ng - 1));
+    constexpr int c0 = FF ? kFoldBias : 0;
+#pragma unroll
+    for (int j = 0; j < WN; ++j) {
+      const v4i B0 = unpack_b<BITS, FF>(o.B[0][j]), B1 = unpack_b<BITS, FF>(o.B[1][j]);
+      const uint32_t zw = o.z[j];
+      fetch(o, j, min(g + 2, ng - 1));
+      v4i T[WM];
+#pragma unroll
+      for (int i = 0; i < WM; ++i)
+        T[i] = __builtin_amdgcn_mfma_i32_16x16x64_i8(A[0][i], B0, (v4i){c0, c0, c0, c0}, 0, 0, 0);
+#pragma unroll
+      for (int i = 0; i < WM; ++i) T[i] = __builtin_amdgcn_mfma_i32_16x16x64_i8(A[1][i], B1, T[i], 0, 0, 0);
+      const float sc = ifrd::h2f((uint16_t)(zw & 0xFFFFu)), h = 0.5f * sc;
+      const float ze = ifrd::h2f((uint16_t)(zw >> 16));
+#pragma unroll
+      for (int i = 0; i < WM; ++i)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          if constexpr (FF) {
+            acc[i][j][r] = fmaf(h, __int_as_float(T[i][r]) - S[i][r], acc[i][j][r]);
+          } else {
+            const int32_t Tv = true_t<BITS>(T[i][r], S[i][r]);
+            acc[i][j][r] = fmaf(sc, fmaf(-ze, S[i][r], (float)Tv), acc[i][j][r]);
+          }
+        }
+    }
+    __syncthreads();
+  };
+  for (int g = 0;; g += 2) {
+    group(g, ring[0]);
+    if (g + 1 >= ng) break;
+    group(g + 1, ring[1]);
+    if (g + 2 >= ng) break;
+  }
+  float asr[WM][4];
+#pragma unroll
+  for (int i = 0; i < WM; ++i)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) asr[i][r] = p.as[min(bm0 + 16 * i + 4 * lgrp + r, p.M - 1)] * p.post;
+  store_tiles<WM, WN, EPI, false>(p, lds_f, acc, asr, bm0, tile0, wave, lane);
+}
+
 // ---- small M (decode, weight-stream bound): the 4 waves split the K groups
 // of one WM x WN tile block.  Each wave issues the loads of all its groups
 // (at most NGW) at entry, runs the MFMAs, and parks its int32 T in LDS; after
@@ -1391,6 +1556,44 @@ hipError_t launch_full_ng(const KParams& p, hipStream_t st) {
   }
 }
 
+template <int BITS, int WM, int WN, int EPI>
+hipError_t launch_tall(const KParams& p, hipStream_t st) {
+  constexpr int BM = 16 * WM, BN = 64 * WN;
+  if constexpr (WN * BITS > 16) {  // two groups of codes would not fit the registers
+    return hipErrorInvalidValue;
+  } else {
+    const size_t lds = std::max((size_t)4 * WM * 1024 + (size_t)p.ng * (BM + 4) * sizeof(float),
+                                (size_t)4 * BM * (EPI == 0 ? 16 * WN : 8 * WN) * sizeof(uint16_t));
+    if (p.tdump || lds > 160 * 1024) return hipErrorInvalidValue;
+    constexpr bool kFF = BITS != 8;
+    static bool attr_set = false;
+    if (!attr_set) {
+      hipError_t e = set_lds_limit(qgemm_tall<BITS, WM, WN, EPI, false>);
+      if constexpr (kFF)
+        if (e == hipSuccess) e = set_lds_limit(qgemm_tall<BITS, WM, WN, EPI, true>);
+      if (e != hipSuccess) return e;
+      attr_set = true;
+    }
+    KParams q = p;
+    q.vst = reinterpret_cast<uintptr_t>(p.out) % 16 == 0 && p.ldo % 8 == 0;
+    q.nbx = (p.N / 16 + BN / 16 - 1) / (BN / 16);
+    q.nby = (p.M + BM - 1) / BM;
+    // the column order of launch_rows, by the same rule
+    const size_t colblock_bytes = (size_t)BN * p.K * BITS / 8 + (size_t)BN * p.ng * 4;
+    const size_t mb2 = (size_t)2 << 20, mb3 = (size_t)3 << 20;
+    q.swz = (q.nbx >= 8 && q.nby >= 2 && (size_t)((q.nbx + 7) / 8) * colblock_bytes > mb3)
+                ? (int)std::max<size_t>(1, mb2 / colblock_bytes) : 0;
+    const dim3 grid = q.swz > 0 ? dim3((q.nbx + 7) / 8 * 8 * q.nby) : dim3(q.nbx, q.nby);
+    if constexpr (kFF)
+      if (p.ff) {
+        hipLaunchKernelGGL((qgemm_tall<BITS, WM, WN, EPI, true>), grid, dim3(256), lds, st, q);
+        return hipGetLastError();
+      }
+    hipLaunchKernelGGL((qgemm_tall<BITS, WM, WN, EPI, false>), grid, dim3(256), lds, st, q);
+    return hipGetLastError();
+  }
+}
+
 template <int BITS, int WM, int WN, int MW, int EPI>
 hipError_t launch_full(const KParams& p, hipStream_t st) {
   if constexpr (BITS == 8) {
@@ -1455,13 +1658,33 @@ hipError_t launch_bits(const KParams& p, int variant, hipStream_t st) {
     const int splitk_max = narrow ? (p.ng <= 16 ? 576 : 256) : 128;
     if (p.ng <= 24 && p.M <= splitk_max) variant = 0;
     else variant = narrow ? 4 : 5;
-    // The 27B-class shapes (K >= 4096; bench.py --gemm-variants-27b, M = 512
-    // and 2160): the 136-group down projection keeps its A and B tiles
-    // resident best in 64 x 64 blocks, 128 x 64 from M = 1024 (M = 2160:
-    // 465 -> 449 us); the others gain from 32 x 256 once M or N is large.
-    if (p.K >= 4096 && p.M > 256) {
-      if (p.ng >= 96) variant = p.M >= 1024 ? 9 : 3;
-      else if (p.M >= 1024 || p.N >= 6144) variant = 6;
+    // The wide shapes (K >= 4096), M > 16 (K = 5120 and 17408, N = 5120, 7168
+    // and 2 x 17408, M = 17 .. 2160, us).  While the 64 x 64 blocks fit one
+    // round of the CUs they win by their shorter groups (K 5120 N 5120, M =
+    // 128: 15.2 against 21.6 of 32 x 128 and 32.1 of the tall 64 x 128), then
+    // 128 x 64 the same way (K 17408, M = 384: 85.5 against 97.2 of 64 x 64
+    // and 100.4 tall); beyond that the tall blocks, whose time per CU is
+    // about 31, 36 and 48 us for 1, 2 and 3 of 64 x 128 and 48 and 59 us for
+    // 1 and 2 of 64 x 256, in these rounds (M = 1024, N 5120: 48.2 and 59.5;
+    // N 7168: 73.7 and 59.3).  Up to 32 rows the 64-row blocks are half
+    // empty: the wide pair keeps 32 x 128 (M = 32: 30.1 against 37.2).
+    if (p.K >= 4096 && p.M > 16) {
+      auto blocks = [&](long bm, long bn) { return ((p.M + bm - 1) / bm) * ((p.N + bn - 1) / bn); };
+      int tall = -1;
+      if (blocks(64, 64) <= 256) variant = 3;
+      else if (blocks(128, 64) <= 256) variant = 9;
+      else if (p.M > 32) {
+        const long n21 = (blocks(64, 128) + 255) / 256, n22 = (blocks(64, 256) + 255) / 256;
+        const long t21 = 48 * (n21 / 3) + (n21 % 3 == 0 ? 0 : n21 % 3 == 1 ? 31 : 36);
+        const long t22 = 59 * (n22 / 2) + 48 * (n22 % 2);
+        tall = t22 < t21 ? 22 : 21;
+      }
+      if (tall >= 0) {  // a shape they cannot hold keeps the choice above
+        hipError_t e = launch_bits<BITS, EPI>(p, tall, st);
+        if (e == hipErrorInvalidValue && tall == 22) e = launch_bits<BITS, EPI>(p, 21, st);
+        if (e != hipErrorInvalidValue) return e;
+        if (p.M > 256) variant = p.ng >= 96 ? (p.M >= 1024 ? 9 : 3) : p.M >= 1024 || p.N >= 6144 ? 6 : variant;
+      }
     }
     // The mixed-iteration shapes (K of 8, 16 or 24 groups, 128 < M <= 1024;
     // bench.py --gemm-variants --gemm-mall, weights MALL-resident as in the
@@ -1526,6 +1749,8 @@ hipError_t launch_bits(const KParams& p, int variant, hipStream_t st) {
     case 18: return launch_full<BITS, 1, 2, 1, EPI>(p, st);           // 16 x 128 block
     case 19: return launch_full<BITS, 2, WNs, 1, EPI>(p, st);         // 32 x 64 block
     case 20: return launch_full<BITS, 1, WNs, 2, EPI>(p, st);         // 32 x 32 block
+    case 21: return launch_tall<BITS, 4, 2, EPI>(p, st);              // 64 x 128 block, 64 x 32 per wave
+    case 22: return launch_tall<BITS, 4, 4, EPI>(p, st);              // 64 x 256 block, 64 x 64 per wave
     default: return hipErrorInvalidValue;
   }
 }

@@ -456,3 +456,50 @@ def test_pack_maps_match_restatement(dev, case):
     # every unit is dispatched exactly once
     live = sorted(u for u in exp["order"] if u >= 0)
     assert live == list(range(nu.value))
+
+
+@pytest.mark.parametrize("bits,zmode", [(2, "codebook"), (4, "codebook"), (8, "codebook"), (2, "general")])
+def test_qgemm_tall_blocks_odd_depths(dev, bits, zmode):
+    """The tall blocks (64 rows per wave) at odd group counts, one group,
+    partial row blocks and column tiles, against the oracle; and the default
+    choice where it takes them (K >= 4096, more 128 x 64 blocks than CUs)
+    against the 64 x 64 shape."""
+    rng = np.random.default_rng(700 + bits)
+    nv = L.ifr_quant_gemm_variants()
+
+    def run(N, K, Ms, check):
+        zero = None if zmode == "codebook" else rng.uniform(0, (1 << bits) - 1, size=(N, K // 128))
+        lin = ia.make_linear(N, K, bits, rng, zero=zero)
+        dl = C.c_void_p()
+        ia.check(L.ifr_linear_upload(dev.ctx, C.byref(lin.struct), C.byref(dl)), "upload")
+        try:
+            for M in Ms:
+                q, sc, g = po.act_quant(rng.standard_normal((M, K), dtype=np.float32))
+                qd, sd, gd = dev.upload(ia.atile(q)), dev.upload(sc[:, 0].copy()), dev.upload(g)
+                od = dev.alloc(M * N * 2)
+                announce(f"tall blocks bits={bits} {zmode} N={N} K={K} M={M}")
+                check(lin, dl, q, sc, (qd.p, sd.p, gd.p, M, od.p), lambda: dev.download(od, np.uint16, (M, N)))
+                for b in (qd, sd, gd, od):
+                    b.free()
+        finally:
+            L.ifr_linear_free(dev.ctx, dl)
+
+    def vs_oracle(lin, dl, q, sc, args, out):
+        ref = po.qgemm(q, sc[:, 0], lin)
+        for v in (nv - 2, nv - 1):
+            rc = L.ifr_quant_gemm_variant(dev.ctx, dl, *args, v)
+            if bits == 8 and v == nv - 1:
+                assert rc == ia.IFR_EDECLINE
+                continue
+            ia.check(rc, f"variant {v}")
+            assert np.array_equal(out(), ref), (v, q.shape)
+
+    def vs_blocks(lin, dl, q, sc, args, out):
+        ia.check(L.ifr_quant_gemm_variant(dev.ctx, dl, *args, 3), "64 x 64")
+        ref = out()
+        ia.check(L.ifr_quant_gemm(dev.ctx, dl, *args, None), "default")
+        assert np.array_equal(out(), ref), q.shape
+
+    run(80, 128, (1, 64, 65), vs_oracle)
+    run(336, 384, (63, 130), vs_oracle)
+    run(16448, 4224, (33, 200), vs_blocks)
