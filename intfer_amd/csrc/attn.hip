@@ -353,26 +353,18 @@ __global__ __launch_bounds__(256) void attn_kernel(AttnArgs p, KVLayout kv) {
 
 // Merge the KV-split partials of one row for all heads, then per-token int8
 // quantization (half-away) of the [nq*hd] attention row for the O projection.
-// Thread t owns the CS consecutive dims [CS t, CS t + CS) of the row (CS a
-// power of two dividing hd, so a chunk never straddles a head; threads past
-// nq*hd/CS idle).  The merge runs the splits in order: the max over all
-// splits first, then l and O accumulated split by split, loaded in rounds of
-// 4 with clamped (unconditional) indices so each round is one memory latency.
-template <int CS>
-__device__ __forceinline__ int group_sum_int(int v) {
-  // the 128 columns of one K group are 128 / CS consecutive lanes
-  if constexpr (CS == 8) {
-    return ifrd::row16_sum_int(v);
-  } else {
-    v += __builtin_bit_cast(int, ifrd::lane_xor<1>(__builtin_bit_cast(float, v)));
-    v += __builtin_bit_cast(int, ifrd::lane_xor<2>(__builtin_bit_cast(float, v)));
-    if constexpr (CS == 16) v += __builtin_bit_cast(int, ifrd::lane_xor<4>(__builtin_bit_cast(float, v)));
-    return v;
-  }
-}
-
-template <int CS>
-__global__ __launch_bounds__(256) void combine_kernel(CombineArgs a) {
+// Thread t owns the 8 consecutive dims [8 t, 8 t + 8) of the row (a chunk never
+// straddles a head; threads past nq*hd/8 idle), 256 threads up to 2048 columns,
+// 640 up to 5120, else 1024.  Bound by the latency of its dependent loads, so
+// a wide row gets more threads and not more columns a thread (40 heads, 60
+// rows: 32 columns a thread in 256 threads, two rounds of loads at 208 VGPRs,
+// 20.1 us; 640 threads 9.8 us).
+// The merge runs the splits in order: the max over all splits first, then l
+// and O accumulated split by split, loaded in rounds of 4 with clamped
+// (unconditional) indices so each round is one memory latency.
+template <int NT>
+__global__ __launch_bounds__(NT) void combine_kernel(CombineArgs a) {
+  constexpr int CS = 8, NW = NT / 64;
   const int m = blockIdx.x;
   const int N = a.nq * a.hd;
   const int G = a.nq / a.nkv;
@@ -402,7 +394,7 @@ __global__ __launch_bounds__(256) void combine_kernel(CombineArgs a) {
   // Up to R1 splits: one round of loads, the max taken from the loaded
   // (m, l) pairs; more: a max pass, then the weighted sum.  Either way the
   // splits are summed in ascending order with the same operands.
-  constexpr int R1 = CS == 8 ? 8 : 4;
+  constexpr int R1 = 8;
   if (ns <= R1) {
     float2 mlv[R1];
     float4 ov[R1][CS / 4];
@@ -463,7 +455,7 @@ __global__ __launch_bounds__(256) void combine_kernel(CombineArgs a) {
     }
   }
   const float invL = 1.0f / L;
-  __shared__ float red[4];
+  __shared__ float red[NW];
   float amax = 0.0f;
 #pragma unroll
   for (int i = 0; i < CS; ++i) {
@@ -480,11 +472,13 @@ __global__ __launch_bounds__(256) void combine_kernel(CombineArgs a) {
   amax = ifrd::wave_max(amax);
   if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = amax;
   __syncthreads();
-  const float mxa = fmaxf(1e-6f, fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3])));
+  float mxa = 1e-6f;
+#pragma unroll
+  for (int i = 0; i < NW; ++i) mxa = fmaxf(mxa, red[i]);
   const float sc = mxa / 127.0f;
   const float inv = 1.0f / sc;
   if (threadIdx.x == 0) a.qscale[m] = sc;
-  // CS consecutive columns sit in one or two 16-byte A-tile lane chunks
+  // 8 consecutive columns sit in one 16-byte A-tile lane chunk
   uint32_t w[CS / 4];
   int csum = 0;
 #pragma unroll
@@ -495,16 +489,9 @@ __global__ __launch_bounds__(256) void combine_kernel(CombineArgs a) {
     w[i >> 2] |= (uint32_t)(c & 0xFF) << (8 * (i & 3));
     csum += c;
   }
-  csum = group_sum_int<CS>(csum);
+  csum = ifrd::row16_sum_int(csum);  // the 128 columns of a K group are 16 consecutive lanes
   if (!own) return;
-  if constexpr (CS == 8) {
-    *reinterpret_cast<uint2*>(a.q + atile_off(m, e0, N)) = make_uint2(w[0], w[1]);
-  } else {
-#pragma unroll
-    for (int r = 0; r < CS / 16; ++r)
-      *reinterpret_cast<uint4*>(a.q + atile_off(m, e0 + 16 * r, N)) =
-          make_uint4(w[4 * r], w[4 * r + 1], w[4 * r + 2], w[4 * r + 3]);
-  }
+  *reinterpret_cast<uint2*>(a.q + atile_off(m, e0, N)) = make_uint2(w[0], w[1]);
   if (threadIdx.x % (128 / CS) == 0) a.gsum[(size_t)m * (N / 128) + e0 / 128] = (float)csum;
 }
 
@@ -534,9 +521,9 @@ hipError_t launch_combine(const CombineArgs& a, hipStream_t st) {
   const int N = a.nq * a.hd;
   if (N % 128 != 0 || N > 256 * 32 || a.hd != kHD || !a.q || !a.qscale || !a.gsum)
     return hipErrorInvalidValue;
-  if (N <= 256 * 8) hipLaunchKernelGGL(combine_kernel<8>, dim3(a.M), dim3(256), 0, st, a);
-  else if (N <= 256 * 16) hipLaunchKernelGGL(combine_kernel<16>, dim3(a.M), dim3(256), 0, st, a);
-  else hipLaunchKernelGGL(combine_kernel<32>, dim3(a.M), dim3(256), 0, st, a);
+  if (N <= 256 * 8) hipLaunchKernelGGL(combine_kernel<256>, dim3(a.M), dim3(256), 0, st, a);
+  else if (N <= 640 * 8) hipLaunchKernelGGL(combine_kernel<640>, dim3(a.M), dim3(640), 0, st, a);
+  else hipLaunchKernelGGL(combine_kernel<1024>, dim3(a.M), dim3(1024), 0, st, a);
   return hipGetLastError();
 }
 

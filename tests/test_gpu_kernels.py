@@ -5,6 +5,7 @@ act-quant codes/scales/group sums, the packing maps.  Tolerance: attention
 (fp16 P in the PV MFMA, online softmax), SwiGLU (device expf).
 """
 import ctypes as C
+import sys
 from concurrent.futures import ThreadPoolExecutor
 
 import numpy as np
@@ -503,3 +504,41 @@ def test_qgemm_tall_blocks_odd_depths(dev, bits, zmode):
     run(80, 128, (1, 64, 65), vs_oracle)
     run(336, 384, (63, 130), vs_oracle)
     run(16448, 4224, (33, 200), vs_blocks)
+
+
+@pytest.mark.parametrize("heads", [24, 48, 64])
+def test_attention_row_widths(dev, heads):
+    """Rows of 3072, 6144 and 8192 attention columns (the combine's 640- and
+    1024-thread rows, partly idle and full), short and beyond the 8 KV splits
+    merged in one round."""
+    cfg = ia.default_cfg(layers=1, vocab=512, hidden=256, inter=256, n_heads=heads)
+    lens, model = [5, 2305, 700], ia.SynthModel(cfg, seed=5)
+    eng = ia.Engine(dev, model, max_seqs=4, max_seq_tokens=4096, max_rows=16)
+    rng = np.random.default_rng(heads)
+    nkv, hd, seqs, kvs = cfg.n_kv, cfg.head_dim, [], []
+    for n in lens:
+        seqs.append(eng.seq_open())
+        k, v = (rng.standard_normal((1, n, nkv, hd), dtype=np.float32).astype(np.float16).astype(np.float32) for _ in "kv")
+        eng.load_kv(seqs[-1], k, v)
+        kvs.append((k.reshape(n, -1), v.reshape(n, -1)))
+    rows = [(s, n - 1, 0, 0, 1) for s, n in zip(seqs, lens)]
+    q = rng.standard_normal((3, heads, hd), dtype=np.float32).astype(np.float16)
+    announce(f"attention heads={heads}")
+    out = eng.attention(0, rows, q)
+    for m, (n, (k, v)) in enumerate(zip(lens, kvs)):
+        ref = np.zeros(heads * hd, np.float32)
+        po.oracle().or_attention_row(ptr(np.ascontiguousarray(q[m].astype(np.float32))), ptr(k), ptr(v), n - 1, heads,
+                                     nkv, hd, ptr(ref))
+        # fp32 sums over up to 2305 keys with a 2^-22 probability split (test_attention_cfg3 allows 4e-3)
+        assert np.abs(out[m] - ref).max() < 1e-4, m
+    model.close()
+
+
+@pytest.mark.parametrize("M", [1, 2, 256, 257, 512, 513])
+def test_pack_maps_at_small_batch_edges(dev, M, monkeypatch):
+    """The packing maps where the pack kernel's small batch ends (512 rows),
+    where its threads take a second row (256), and at one row."""
+    dec = min(M, 40) if M > 2 else M
+    spec = [(i, 50 + 7 * i, 0, i % 2) for i in range(dec)] + [(dec, 300 + p, 1, int(p == M - dec - 1)) for p in range(M - dec)]
+    monkeypatch.setattr(sys.modules[__name__], "PACK_CASES", [([60 + 7 * i for i in range(dec)] + [900], spec)])
+    test_pack_maps_match_restatement(dev, 0)
