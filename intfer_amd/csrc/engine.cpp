@@ -61,7 +61,8 @@ constexpr int kAttnTiles = 1;  // 16-column MFMA tiles per attention unit (q-blo
 // ---- the no-allocation attention entry point's scratch (ifr_attention_noalloc)
 // Limits of one call: rows, attention units (one per (q-block, kv head,
 // 256-token KV split)) and the attention row width n_heads * head_dim.
-constexpr int kNaRows = 512;
+constexpr int kNaRows = 512;  // (at most kPackSmallRows: their records are read in place)
+static_assert(kNaRows <= ifrk::kPackSmallRows, "");
 constexpr int kNaUnits = 4096;
 constexpr int kNaRowWidth = 8192;
 constexpr size_t na_align(size_t x) { return (x + 255) & ~(size_t)255; }
@@ -522,14 +523,29 @@ int prep_sub(ifr_ctx* c, const ifr_row* rows, SubBatch& sb) {
   return IFR_OK;
 }
 
+// The rows as the pack kernel reads them: into the lane's pinned buffer, and
+// from there read in place up to kPackSmallRows rows (a copy is a launch of its
+// own ahead of the pack kernel, 3 us longer than the read over the bus that
+// replaces it), else through its device copy.  The buffer is free: the lane's last
+// batch was waited for.
+int stage_rows(Lane& L, const ifr_row* r, int M, hipStream_t st, const int32_t** src) {
+  std::memcpy(L.rows_h, r, (size_t)M * sizeof(ifr_row));
+  *src = L.rows_h;
+  if (M > ifrk::kPackSmallRows) {
+    HIPCHK(hipMemcpyAsync(L.rows_d, L.rows_h, (size_t)M * sizeof(ifr_row), hipMemcpyHostToDevice, st));
+    *src = L.rows_d;
+  }
+  return IFR_OK;
+}
+
 // Rows up; the pack kernel writes the packing maps and the token column.
 int launch_head(ifr_ctx* c, const ifr_row* rows, const SubBatch& sb) {
   Lane& L = c->lane[sb.lane];
   const ifr_row* r = rows + sb.row0;
-  std::memcpy(L.rows_h, r, (size_t)sb.M * sizeof(ifr_row));
-  HIPCHK(hipMemcpyAsync(L.rows_d, L.rows_h, (size_t)sb.M * sizeof(ifr_row), hipMemcpyHostToDevice, L.st));
+  const int32_t* src = nullptr;
+  if (int e = stage_rows(L, r, sb.M, L.st, &src)) return e;
   Scope sc(c, L.st, "pack", sb.pack_bytes);
-  HIPCHK(ifrk::launch_pack(L.rows_d, sb.M, c->cfg.n_kv, c->qb, sb.split, L.pk, L.st));
+  HIPCHK(ifrk::launch_pack(src, sb.M, c->cfg.n_kv, c->qb, sb.split, L.pk, L.st));
   return IFR_OK;
 }
 
@@ -1545,9 +1561,9 @@ int ifr_attention(ifr_ctx* c, int32_t layer, const ifr_row* rows, int32_t M, con
   const int nslots = (int)ifrk::attn_slot_count(g_pos0.data(), g_len.data(), (int)g_len.size(), nkv, split,
                                                 c->qb, &nchunked);
   c->last_slots = nslots;
-  std::memcpy(c->lane[0].rows_h, rows, (size_t)M * sizeof(ifr_row));
-  HIPCHK(hipMemcpyAsync(c->lane[0].rows_d, c->lane[0].rows_h, (size_t)M * sizeof(ifr_row), hipMemcpyHostToDevice, c->st));
-  HIPCHK(ifrk::launch_pack(c->lane[0].rows_d, M, nkv, c->qb, split, c->lane[0].pk, c->st));
+  const int32_t* src = nullptr;
+  if (int r = stage_rows(c->lane[0], rows, M, c->st, &src)) return r;
+  HIPCHK(ifrk::launch_pack(src, M, nkv, c->qb, split, c->lane[0].pk, c->st));
   HIPCHK(hipMemcpyAsync(c->lane[0].qbuf, q_h, (size_t)M * nq * hd * 2, hipMemcpyHostToDevice, c->st));
   ifrk::KVLayout kv{nkv, hd, kPage, c->max_pages, c->kv.kv_int8, c->kpool[layer], c->vpool[layer],
                     c->kscale[layer], c->vscale[layer], c->bt_d};
@@ -1618,8 +1634,13 @@ int ifr_attention_noalloc(ifr_ctx* c, int32_t layer, const ifr_row* rows, int32_
   // every region is fully written by the kernel that produces it before it
   // is read (the pack maps, each unit's partials, the combine outputs), so
   // nothing is cleared between calls
-  HIPCHK(hipMemcpyAsync(rows_d, rows, (size_t)M * sizeof(ifr_row), hipMemcpyHostToDevice, c->st));
-  HIPCHK(ifrk::launch_pack(rows_d, M, nkv, c->qb, split, pk, c->st));
+  const int32_t* src = rows_d;
+  if (M <= c->maxM) {
+    if (int r = stage_rows(c->lane[0], rows, M, c->st, &src)) return r;
+  } else {  // more rows than the engine's own buffers hold
+    HIPCHK(hipMemcpyAsync(rows_d, rows, (size_t)M * sizeof(ifr_row), hipMemcpyHostToDevice, c->st));
+  }
+  HIPCHK(ifrk::launch_pack(src, M, nkv, c->qb, split, pk, c->st));
   ifrk::KVLayout kv{nkv, hd, kPage, c->max_pages, c->kv.kv_int8, c->kpool[layer], c->vpool[layer],
                     c->kscale[layer], c->vscale[layer], c->bt_d};
   ifrk::AttnArgs a{pk.units, (int)nunits, pk.order, (int)nslots, shared_slots(c, nchunked), q_d, nq,
@@ -1629,7 +1650,7 @@ int ifr_attention_noalloc(ifr_ctx* c, int32_t layer, const ifr_row* rows, int32_
                        reinterpret_cast<int8_t*>(S + kNaAqOff), reinterpret_cast<float*>(S + kNaAsOff),
                        reinterpret_cast<float*>(S + kNaGsOff), 16 * kAttnTiles};
   HIPCHK(ifrk::launch_combine(cb, c->st));
-  // the rows copy read the caller's host array; return once out_d is written
+  // the rows are read from host memory; return once out_d is written
   HIPCHK(hipStreamSynchronize(c->st));
   return IFR_OK;
 }

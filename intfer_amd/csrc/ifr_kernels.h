@@ -230,8 +230,11 @@ struct PackOut {
 // *chunked receives the size of the chunked region (a multiple of 4).
 long attn_slot_count(const int* g_pos0, const int* g_len, int ngroups, int nkv, int split, int qb,
                      long* chunked = nullptr);
-// rows: device copy of ifr_row[M] (5 int32 each).  qb = q-block tokens,
-// split = kv tokens per unit (multiple of the page size).
+// rows: ifr_row[M] (5 int32 each) in device memory or, up to
+// kPackSmallRows rows, in pinned host memory (each of the launch's 4 workgroups
+// reads the records once, in order).  qb = q-block tokens, split = kv tokens
+// per unit (multiple of the page size).
+constexpr int kPackSmallRows = 512;
 hipError_t launch_pack(const int32_t* rows, int M, int nkv, int qb, int split, const PackOut& o,
                        hipStream_t st);
 

@@ -933,12 +933,12 @@ __device__ __forceinline__ int pack_group_of(const uint16_t* nblk, int ngroups, 
   return lo;
 }
 
-// kPackGroups workgroups of kPackThreads.  Each builds the whole set of maps
-// in its own LDS (the batch is at most 6144 rows), and the workgroups share
-// the writes: workgroup g stores the per-row outputs of the rows its wave g
-// holds, and every kPackGroups-th (q-block, kv head) pair's units and
-// dispatch slots.  Row m = threadIdx.x + k kPackThreads is read from global
-// memory once, into registers (k < kPackRowsPerThread); every later phase
+// T / 64 workgroups of T threads (1024; 256 up to 512 rows).  Each builds the
+// whole set of maps in its own LDS (the batch is at most 6144 rows), and the
+// workgroups share the writes: workgroup g stores the per-row outputs of the
+// rows its wave g holds, and every (T / 64)-th (q-block, kv head) pair's units
+// and dispatch slots.  Row m = threadIdx.x + k T is read from global memory
+// once, into registers (k < R = kPackRowsPerThread); every later phase
 // works from those registers and six LDS arrays, and every loop runs over
 // rows, groups or q-blocks in parallel (no thread walks a group's q-blocks
 // or quads).  Ten barriers in all.  LDS arrays, one map per phase (the
@@ -952,36 +952,58 @@ __device__ __forceinline__ int pack_group_of(const uint16_t* nblk, int ngroups, 
 //   nblk    first q-block of group g (nb at ngroups)    16 bits
 //   bgrp    group of q-block b                          16 bits
 constexpr int kPackThreads = 1024, kPackRowsPerThread = 6, kPackMaxRows = kPackThreads * kPackRowsPerThread;
-constexpr int kPackGroups = 16;
+// The ten barriers and the chain of loads and stores between them are what a
+// small batch waits for (6.8 us at one row, 7.7 at 512), not its work, so up to
+// 512 rows 4 workgroups of 4 waves take it and read each record once, in order,
+// through LDS: the records can then stay in host memory, without the copy
+// ahead of the launch (attention on one decode row 33.9 -> 31.2 us a call, on a
+// 512-row chunk 51.9 -> 50.0; with the copy kept 34.3 and 51.5).
+constexpr int kPackSmallThreads = 256;
 static_assert(kPackMaxRows < 65536, "the 16-bit index maps hold row, group and q-block indices");
 
-__global__ __launch_bounds__(kPackThreads) void pack_kernel(const int32_t* rows, int M, int nkv, int qb,
-                                                            int split, PackOut o) {
+template <int T, int R, bool STAGE>
+__global__ __launch_bounds__(T) void pack_kernel(const int32_t* rows, int M, int nkv, int qb, int split, PackOut o) {
+  constexpr int NG = T / 64;  // workgroups
   extern __shared__ int sm[];
   int* fs = sm;                  // [M]
   int* fw = sm + M;              // [M]
   int* gpos = sm + 2 * M;        // [M]
   int* gseq = sm + 3 * M;        // [M]
   int* ucnt = sm + 4 * M;        // [M]
-  int* tmp = sm + 5 * M;         // [2 kPackThreads / 64]
-  uint16_t* g0 = reinterpret_cast<uint16_t*>(tmp + 2 * kPackThreads / 64);  // [M + 1]
+  int* tmp = sm + 5 * M;         // [2 T / 64]
+  uint16_t* g0 = reinterpret_cast<uint16_t*>(tmp + 2 * T / 64);  // [M + 1]
   uint16_t* nblk = g0 + M + 1;   // [M + 1]
   uint16_t* bgrp = nblk + M + 1; // [M]
-  constexpr int R = kPackRowsPerThread;
   // this workgroup's share of the writes: pairs t0, t0 + tstep, ... (64
   // consecutive pairs per wave: a store instruction costs about the same
   // whether 4 or 64 of its lanes are active); the rows of wave wg
-  const int wg = blockIdx.x, t0 = wg + kPackGroups * threadIdx.x, tstep = kPackGroups * kPackThreads;
+  const int wg = blockIdx.x, t0 = wg + NG * threadIdx.x, tstep = NG * T;
   const bool rows_out = (int)(threadIdx.x >> 6) == wg;
   // KV splits of a q-block of group g ending at its block b (q-block rows up to (b + 1) qb)
   auto nsplit = [&](int g, int b) {
     return (gpos[g] + min((b + 1) * qb, g0[g + 1] - g0[g]) + split - 1) / split;
   };
+  if constexpr (STAGE) {  // the records as consecutive dwords into the first five LDS arrays
+    constexpr int Q = 5 * R;
+    int x[Q];
+#pragma unroll
+    for (int q = 0; q < Q; ++q) {
+      const int i = threadIdx.x + q * T;
+      x[q] = i < 5 * M ? rows[i] : 0;
+    }
+#pragma unroll
+    for (int q = 0; q < Q; ++q) {
+      const int i = threadIdx.x + q * T;
+      if (i < 5 * M) sm[i] = x[q];
+    }
+    __syncthreads();
+    rows = sm;
+  }
   int seq_r[R], pos_r[R], g_r[R];
   bool start_r[R], want_r[R];
 #pragma unroll
   for (int k = 0; k < R; ++k) {
-    const int m = threadIdx.x + k * kPackThreads;
+    const int m = threadIdx.x + k * T;
     start_r[k] = want_r[k] = false;
     seq_r[k] = pos_r[k] = g_r[k] = 0;
     if (m < M) {
@@ -992,14 +1014,21 @@ __global__ __launch_bounds__(kPackThreads) void pack_kernel(const int32_t* rows,
       pos_r[k] = pos;
       start_r[k] = st;
       want_r[k] = want != 0;
-      fs[m] = st ? 1 : 0;
-      fw[m] = want ? 1 : 0;
       if (rows_out) {
         o.row_seq[m] = seq;
         o.row_pos[m] = pos;
         o.row_kind[m] = kind;
         if (o.row_tok) o.row_tok[m] = tok;
       }
+    }
+  }
+  if constexpr (STAGE) __syncthreads();  // the staged records are read: their LDS holds the maps from here on
+#pragma unroll
+  for (int k = 0; k < R; ++k) {
+    const int m = threadIdx.x + k * T;
+    if (m < M) {
+      fs[m] = start_r[k] ? 1 : 0;
+      fw[m] = want_r[k] ? 1 : 0;
     }
   }
   __syncthreads();
@@ -1012,7 +1041,7 @@ __global__ __launch_bounds__(kPackThreads) void pack_kernel(const int32_t* rows,
   // position and sequence of each group
 #pragma unroll
   for (int k = 0; k < R; ++k) {
-    const int m = threadIdx.x + k * kPackThreads;
+    const int m = threadIdx.x + k * T;
     if (m < M) {
       const int g = fs[m] + (start_r[k] ? 1 : 0) - 1;
       g_r[k] = g;
@@ -1030,7 +1059,7 @@ __global__ __launch_bounds__(kPackThreads) void pack_kernel(const int32_t* rows,
   if (threadIdx.x == 0) g0[ngroups] = (uint16_t)M;
   __syncthreads();
   if (wg == 0)
-    for (int g = threadIdx.x; g <= ngroups; g += kPackThreads) o.cu_seqlens[g] = g0[g];
+    for (int g = threadIdx.x; g <= ngroups; g += T) o.cu_seqlens[g] = g0[g];
   uint16_t* const sblk[1] = {nblk};
   const int nb = block_exscan_f<1, uint16_t>(sblk, ngroups, true, tmp, [&](int g, int (&x)[1]) {
     x[0] = (g0[g + 1] - g0[g] + qb - 1) / qb;  // q-blocks of group g
@@ -1066,7 +1095,7 @@ __global__ __launch_bounds__(kPackThreads) void pack_kernel(const int32_t* rows,
   // each row's combine map (q-block gb = its group's first block + (m - r0) / qb)
 #pragma unroll
   for (int k = 0; k < R; ++k) {
-    const int m = threadIdx.x + k * kPackThreads;
+    const int m = threadIdx.x + k * T;
     if (m < M && rows_out) {
       const int g = g_r[k], r0 = g0[g], len = g0[g + 1] - r0, pos0 = gpos[g];
       const int b = (m - r0) / qb, gb = nblk[g] + b;
@@ -1262,15 +1291,25 @@ hipError_t launch_pack(const int32_t* rows, int M, int nkv, int qb, int split, c
                        hipStream_t st) {
   if (M <= 0) return hipSuccess;
   if (M > kPackMaxRows || qb <= 0 || split <= 0 || nkv <= 0) return hipErrorInvalidValue;
-  const size_t lds = (size_t)(5 * M + 2 * kPackThreads / 64) * sizeof(int) + (size_t)(3 * M + 2) * sizeof(uint16_t);
+  auto lds = [&](int T) {
+    return (size_t)(5 * M + 2 * T / 64) * sizeof(int) + (size_t)(3 * M + 2) * sizeof(uint16_t);
+  };
+  if (M <= kPackSmallRows) {
+    constexpr int T = kPackSmallThreads;
+    hipLaunchKernelGGL((pack_kernel<T, kPackSmallRows / T, true>), dim3(T / 64), dim3(T), lds(T), st, rows, M, nkv, qb,
+                       split, o);
+    return hipGetLastError();
+  }
+  constexpr int T = kPackThreads;
   static bool attr = false;
   if (!attr) {
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(pack_kernel),
+    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(pack_kernel<T, kPackRowsPerThread, false>),
                                        hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
     if (e != hipSuccess) return e;
     attr = true;
   }
-  hipLaunchKernelGGL(pack_kernel, dim3(kPackGroups), dim3(kPackThreads), lds, st, rows, M, nkv, qb, split, o);
+  hipLaunchKernelGGL((pack_kernel<T, kPackRowsPerThread, false>), dim3(T / 64), dim3(T), lds(T), st, rows, M, nkv, qb,
+                     split, o);
   return hipGetLastError();
 }
 
