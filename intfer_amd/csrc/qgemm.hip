@@ -1319,6 +1319,209 @@ __global__ __launch_bounds__(64 * NWV) void qgemm_stream(KParams p) {
   }
 }
 
+// ---- few rows on deep weights (K >= 4096): split K in turns.  A workgroup of
+// NWV waves owns a 16 WM x 16 WN block of outputs; in turn t wave w takes K
+// group t NWV + w: MFMAs, d of the fold, d parked in LDS; after the turn's one
+// barrier WM WN of the waves fold one 16 x 16 tile each over the turn's groups,
+// ascending, so the accumulators stay in registers and the bits are those of
+// every other shape.  The row-block shapes walk the 40 to 136 groups one by one
+// on as many CUs as there are blocks, each group a memory and MFMA latency
+// (down 17408 -> 5120 at 64 rows: 136 groups, 80 blocks, 51 us); here a turn
+// costs about one of their groups.  Bound by LDS traffic (each d written and
+// read once: 16 KB a group at 64 x 32).  The codes of four turns and the A rows
+// of two are in flight in registers; S (FF: the MFMA's start value, whose bits
+// make the result read as 1.5 * 2^23 + 2T - C S) and the scale | zero pairs
+// of a turn are staged in LDS, four buffers.
+// Down 17408 -> 5120, INT2, 32 rows 47.4 -> 17.7 us, 16 rows (16 waves) 20.3 ->
+// 12.7; O 5120 -> 5120, 32 rows 13.9 -> 7.8.
+template <int BITS, int WM, int WN, int NWV, int EPI, bool FF>
+__global__ __launch_bounds__(64 * NWV) void qgemm_turns(KParams p) {
+  constexpr int BM = 16 * WM, BN = 16 * WN, TT = WM * WN, NT = 64 * NWV, SP = BM + 4;
+  static_assert(TT <= NWV && BM * NWV <= NT && BN * NWV <= NT, "one tile per folding wave, one staged value per thread");
+  constexpr int RB = 4, RA = 2;  // turns of weights, of A and S in flight
+  extern __shared__ v4f lds_f4[];
+  v4f* const D_l = lds_f4;                                               // [2][NWV][TT][64]
+  uint32_t* const S_l = reinterpret_cast<uint32_t*>(D_l + 2 * NWV * TT * 64);  // [4][NWV][SP]
+  uint32_t* const Z_l = S_l + 4 * NWV * SP;                              // [4][NWV][BN]
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lrow = lane & 15, lgrp = lane >> 4;
+  const int ntiles = p.N >> 4, ng = p.ng, nturn = (ng + NWV - 1) / NWV;
+  const int bm0 = blockIdx.y * BM, tile0 = blockIdx.x * WN;
+  int tl[WN];
+#pragma unroll
+  for (int j = 0; j < WN; ++j) tl[j] = min(tile0 + j, ntiles - 1);
+  uint32_t at[WM];  // first 1 KB A tile of each row tile (past the last one: the last, never stored)
+#pragma unroll
+  for (int i = 0; i < WM; ++i) at[i] = (uint32_t)(min((bm0 >> 4) + i, (p.M - 1) >> 4) * p.nsteps);
+
+  uint32_t Bw[RB][2][WN][BITS / 2];
+  v4i A[RA][2][WM];
+  auto fetch_b = [&](uint32_t (&B)[2][WN][BITS / 2], int t) {
+    const int g = min(t * NWV + wave, ng - 1);
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int j = 0; j < WN; ++j)
+        load_raw<BITS>(p.codes + ((size_t)tl[j] * p.nsteps + 2 * g + h) * 64 * (BITS / 2), lane, B[h][j]);
+  };
+  auto fetch_a = [&](v4i (&a)[2][WM], int t) {
+    const int g = min(t * NWV + wave, ng - 1);
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int i = 0; i < WM; ++i)
+        a[h][i] = reinterpret_cast<const v4i*>(p.a + (size_t)(at[i] + 2 * g + h) * 1024)[lane];
+  };
+  // a turn's S and scale | zero pairs, one value of each per thread
+  const int sr = threadIdx.x / NWV, sg = threadIdx.x % NWV;
+  const int zc = threadIdx.x % BN, zg = threadIdx.x / BN;
+  float sreg[RA];
+  uint32_t zreg[RB];
+  auto fetch_s = [&](float& v, int t) {
+    if (sr < BM) v = p.gs[(size_t)min(bm0 + sr, p.M - 1) * ng + min(t * NWV + sg, ng - 1)];
+  };
+  auto fetch_z = [&](uint32_t& v, int t) {
+    if (zg < NWV) v = p.sz[((size_t)min(tile0 + (zc >> 4), ntiles - 1) * ng + min(t * NWV + zg, ng - 1)) * 16 + (zc & 15)];
+  };
+  auto store_f = [&](int t, float sv, uint32_t zv) {
+    constexpr int C = (1 << BITS) - 1;
+    if (sr < BM) S_l[((t & 3) * NWV + sg) * SP + sr] = FF ? (uint32_t)(kFoldBias - C * (int)sv) : __float_as_uint(sv);
+    if (zg < NWV)
+      Z_l[((t & 3) * NWV + zg) * BN + zc] = FF ? __float_as_uint(0.5f * ifrd::h2f((uint16_t)(zv & 0xFFFFu))) : zv;
+  };
+  // vector loads return in order, so in every turn the L2-resident A and S
+  // come before the weights: a wait for them then leaves the newer weights out
+#pragma unroll
+  for (int t = 0; t < RB; ++t) {
+    if (t < RA) {
+      fetch_a(A[t], t);
+      fetch_s(sreg[t], t);
+    }
+    fetch_z(zreg[t], t);
+    fetch_b(Bw[t], t);
+  }
+  store_f(0, sreg[0], zreg[0]);
+  fetch_s(sreg[0], 2);
+  fetch_z(zreg[0], RB);
+  // the tile this wave folds
+  const int fi = wave % WM, fj = wave / WM;
+  v4f acc = (v4f){0.f, 0.f, 0.f, 0.f};
+  __syncthreads();
+
+  // sv, zv: the values of turn t + 1
+  auto turn = [&](int t, uint32_t (&B)[2][WN][BITS / 2], v4i (&a)[2][WM], float& sv, uint32_t& zv) {
+    v4f* const D = D_l + (size_t)((t & 1) * NWV) * TT * 64;
+    const int g = t * NWV + wave;
+    if (g < ng) {  // wave-uniform
+      v4i S[WM];
+#pragma unroll
+      for (int i = 0; i < WM; ++i)
+        S[i] = *reinterpret_cast<const v4i*>(&S_l[((t & 3) * NWV + wave) * SP + 16 * i + 4 * lgrp]);
+#pragma unroll
+      for (int j = 0; j < WN; ++j) {
+        const v4i B0 = unpack_b<BITS, FF>(B[0][j]), B1 = unpack_b<BITS, FF>(B[1][j]);
+        const float ze = FF ? 0.f : ifrd::h2f((uint16_t)(Z_l[((t & 3) * NWV + wave) * BN + 16 * j + lrow] >> 16));
+#pragma unroll
+        for (int i = 0; i < WM; ++i) {
+          v4i T = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[0][i], B0, FF ? S[i] : (v4i){0, 0, 0, 0}, 0, 0, 0);
+          T = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[1][i], B1, T, 0, 0, 0);
+          v4f d;
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            if constexpr (FF) {
+              d[r] = __int_as_float(T[r]) - kFoldBiasF;
+            } else {
+              const float Sv = __int_as_float(S[i][r]);
+              d[r] = fmaf(-ze, Sv, (float)true_t<BITS>(T[r], Sv));
+            }
+          }
+          D[(wave * TT + j * WM + i) * 64 + lane] = d;
+        }
+      }
+    }
+    // (buffer (t + 1) & 3 was last read in turn t - 3, three barriers ago)
+    store_f(t + 1, sv, zv);
+    fetch_a(a, t + RA);
+    fetch_s(sv, t + 1 + RA);
+    fetch_z(zv, t + 1 + RB);
+    fetch_b(B, t + RB);
+    __syncthreads();
+    // buffer t & 1 is written again in turn t + 2, behind the barrier of t + 1
+    if (wave < TT) {
+      const int n = min(NWV, ng - t * NWV);
+      const v4f* Dr = D + wave * 64 + lane;
+      const uint32_t* zr = Z_l + (t & 3) * NWV * BN + 16 * fj + lrow;
+      auto fold = [&](int q) {
+        const v4f d = Dr[q * TT * 64];
+        const uint32_t zw = zr[q * BN];
+        const float sc = FF ? __uint_as_float(zw) : ifrd::h2f((uint16_t)(zw & 0xFFFFu));
+#pragma unroll
+        for (int r = 0; r < 4; ++r) acc[r] = fmaf(sc, d[r], acc[r]);
+      };
+      if (n == NWV) {
+#pragma unroll
+        for (int q = 0; q < NWV; ++q) fold(q);
+      } else {
+        for (int q = 0; q < n; ++q) fold(q);
+      }
+    }
+  };
+  for (int t = 0;; t += RB) {
+    turn(t, Bw[0], A[0], sreg[1], zreg[1]);
+    if (t + 1 >= nturn) break;
+    turn(t + 1, Bw[1], A[1], sreg[0], zreg[2]);
+    if (t + 2 >= nturn) break;
+    turn(t + 2, Bw[2], A[0], sreg[1], zreg[3]);
+    if (t + 3 >= nturn) break;
+    turn(t + 3, Bw[3], A[1], sreg[0], zreg[0]);
+    if (t + 4 >= nturn) break;
+  }
+  // the fp16 outputs of the block in LDS (D of the last turn may still be
+  // read), then 16-byte row chunks
+  __syncthreads();
+  uint16_t* const Y = reinterpret_cast<uint16_t*>(lds_f4);  // [BM][BN]
+  if (wave < TT) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int rl = 16 * fi + 4 * lgrp + r;
+      Y[rl * BN + 16 * fj + lrow] = ifrd::f2h(p.as[min(bm0 + rl, p.M - 1)] * p.post * acc[r]);
+    }
+  }
+  __syncthreads();
+  constexpr int TC = EPI == 0 ? BN : BN / 2, CPR = TC / 8;  // output columns of the block, chunks per row
+  const int col0 = EPI == 0 ? 16 * tile0 : 8 * tile0;
+  for (int ch = threadIdx.x; ch < BM * CPR; ch += NT) {
+    const int rl = ch / CPR, cc = (ch % CPR) * 8, row = bm0 + rl;
+    const bool colv = EPI == 0 ? tile0 + cc / 16 < ntiles : tile0 + 2 * (cc / 16) + 1 < ntiles;
+    if (row >= p.M || !colv) continue;
+    uint32_t w[4];
+    if constexpr (EPI == 0) {
+      const uint4 y = *reinterpret_cast<const uint4*>(Y + rl * BN + cc);
+      w[0] = y.x; w[1] = y.y; w[2] = y.z; w[3] = y.w;
+    } else {  // gate tile 2 (cc / 16), up tile next to it
+      const uint16_t* yg = Y + rl * BN + 32 * (cc / 16) + (cc & 15);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        uint32_t o2 = 0;
+#pragma unroll
+        for (int f = 0; f < 2; ++f) {
+          const float gv = ifrd::h2f(yg[2 * e + f]), u = ifrd::h2f(yg[16 + 2 * e + f]);
+          o2 |= (uint32_t)ifrd::f2h(silu_f(gv) * u) << (16 * f);
+        }
+        w[e] = o2;
+      }
+    }
+    uint16_t* dst = p.out + (size_t)row * p.ldo + col0 + cc;
+    if (p.vst) {
+      *reinterpret_cast<uint4*>(dst) = make_uint4(w[0], w[1], w[2], w[3]);
+    } else {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) dst[e] = (uint16_t)(w[e >> 1] >> (16 * (e & 1)));
+    }
+  }
+}
+
 template <typename F>
 hipError_t set_lds_limit(F* f) {
   return hipFuncSetAttribute(reinterpret_cast<const void*>(f), hipFuncAttributeMaxDynamicSharedMemorySize,
@@ -1594,6 +1797,33 @@ hipError_t launch_tall(const KParams& p, hipStream_t st) {
   }
 }
 
+template <int BITS, int WM, int WN, int NWV, int EPI>
+hipError_t launch_turns(const KParams& p, hipStream_t st) {
+  constexpr int BM = 16 * WM, BN = 16 * WN;
+  constexpr size_t lds = (size_t)2 * NWV * WM * WN * 1024 + (size_t)4 * NWV * (BM + 4 + BN) * sizeof(uint32_t);
+  static_assert(lds <= 160 * 1024 && BM * BN * 2 <= 2 * NWV * WM * WN * 1024, "");
+  if (p.tdump) return hipErrorInvalidValue;
+  constexpr bool kFF = BITS != 8;
+  static bool attr_set = false;
+  if (!attr_set) {
+    hipError_t e = set_lds_limit(qgemm_turns<BITS, WM, WN, NWV, EPI, false>);
+    if constexpr (kFF)
+      if (e == hipSuccess) e = set_lds_limit(qgemm_turns<BITS, WM, WN, NWV, EPI, true>);
+    if (e != hipSuccess) return e;
+    attr_set = true;
+  }
+  KParams q = p;
+  q.vst = reinterpret_cast<uintptr_t>(p.out) % 16 == 0 && p.ldo % 8 == 0;
+  const dim3 grid((p.N / 16 + WN - 1) / WN, (p.M + BM - 1) / BM), block(64 * NWV);
+  if constexpr (kFF)
+    if (p.ff) {
+      hipLaunchKernelGGL((qgemm_turns<BITS, WM, WN, NWV, EPI, true>), grid, block, lds, st, q);
+      return hipGetLastError();
+    }
+  hipLaunchKernelGGL((qgemm_turns<BITS, WM, WN, NWV, EPI, false>), grid, block, lds, st, q);
+  return hipGetLastError();
+}
+
 template <int BITS, int WM, int WN, int MW, int EPI>
 hipError_t launch_full(const KParams& p, hipStream_t st) {
   if constexpr (BITS == 8) {
@@ -1670,6 +1900,22 @@ hipError_t launch_bits(const KParams& p, int variant, hipStream_t st) {
     // empty: the wide pair keeps 32 x 128 (M = 32: 30.1 against 37.2).
     if (p.K >= 4096 && p.M > 16) {
       auto blocks = [&](long bm, long bn) { return ((p.M + bm - 1) / bm) * ((p.N + bn - 1) / bn); };
+      // Split K in turns while its blocks are few: 32 x 32 up to one workgroup
+      // per CU, at 2 bits two (INT4's registers allow one, so 64 x 32 there),
+      // and a little further where each row-block group is a longer chain
+      // (136 groups) or the 64-row blocks are half empty (M <= 32).  N 5120,
+      // K 5120: M = 32 13.9 -> 7.8 us, 96 14.3 -> 11.6, 128 14.7 against
+      // 16.3 (row blocks kept); K 17408: M = 32 47.4 -> 17.7, 96 49.1 -> 29.1,
+      // 128 50.4 -> 42.5, 192 54 against 58; the wide pair M = 32 30.6 ->
+      // 27.7; INT4 K 17408: M = 32 59.5 -> 20.5, 64 66.9 -> 34.3.
+      const long b32 = blocks(32, 32);
+      int tv = -1;
+      if (b32 <= 256 || (BITS == 2 && b32 <= (p.ng >= 96 ? 640 : 512)) || (p.M <= 32 && b32 <= 1152)) tv = 24;
+      else if (BITS != 2 && blocks(64, 32) <= 256) tv = 23;
+      if (tv >= 0) {
+        const hipError_t e = launch_bits<BITS, EPI>(p, tv, st);
+        if (e != hipErrorInvalidValue) return e;
+      }
       int tall = -1;
       if (blocks(64, 64) <= 256) variant = 3;
       else if (blocks(128, 64) <= 256) variant = 9;
@@ -1709,15 +1955,22 @@ hipError_t launch_bits(const KParams& p, int variant, hipStream_t st) {
       }
     }
     // Decode rows on those shapes (bench.py --gemm-decode-27b, M = 1, 8, 16):
-    // the weight stream; for the plain projections two tiles per workgroup
-    // up to M = 4, above it one tile (16 waves for the deep down projection,
-    // 8 for the others), and one tile pair of 8 waves for the SwiGLU pair up
-    // to M = 8.  A shape a stream variant cannot hold (registers or LDS for
-    // wider codes) falls back to the next one, then to the choice above.
+    // the weight stream, for the plain projections two tiles per workgroup up
+    // to M = 4 and one above, one tile pair of 8 waves for the SwiGLU pair; its
+    // fold grows with the rows and its parked d with rows and depth, so split K
+    // in turns takes over above 8 rows (M = 16, us: QKV 7.3 -> 6.7, O 7.2 ->
+    // 6.6, gate/up 27.5 -> 21.8, INT4 38.0 -> 28.8) and on the deep down
+    // projection (16 waves) above one row, INT4 above 4 (M = 4 13.4 -> 12.5, 16
+    // 20.3 -> 12.7, M = 1 11.7 against 12.4; INT4 M = 8 20.4 -> 16.8).  A shape
+    // a variant cannot hold (registers or LDS for wider codes) falls back to
+    // the next one, then to the choice above.
     if (p.K >= 4096 && p.M <= 16) {
       hipError_t e = hipErrorInvalidValue;
+      const bool deep = EPI == 0 && p.ng >= 96;
+      if (deep ? p.M > (BITS == 2 ? 1 : 4) : p.M > 8) e = launch_bits<BITS, EPI>(p, deep ? 26 : 25, st);
+      if (e != hipErrorInvalidValue) return e;
       if (EPI == 1) {
-        if (p.M <= 8) e = launch_bits<BITS, EPI>(p, 14, st);
+        e = launch_bits<BITS, EPI>(p, 14, st);
       } else {
         if (p.M <= 4) e = launch_bits<BITS, EPI>(p, 15, st);
         else if (p.ng < 96) e = launch_bits<BITS, EPI>(p, 14, st);
@@ -1751,6 +2004,11 @@ hipError_t launch_bits(const KParams& p, int variant, hipStream_t st) {
     case 20: return launch_full<BITS, 1, WNs, 2, EPI>(p, st);         // 32 x 32 block
     case 21: return launch_tall<BITS, 4, 2, EPI>(p, st);              // 64 x 128 block, 64 x 32 per wave
     case 22: return launch_tall<BITS, 4, 4, EPI>(p, st);              // 64 x 256 block, 64 x 64 per wave
+    // split K in turns, 8 waves: 64, 32 or 16 rows x 32 columns; 16 waves: 16 rows
+    case 23: return launch_turns<BITS, 4, 2, 8, EPI>(p, st);
+    case 24: return launch_turns<BITS, 2, 2, 8, EPI>(p, st);
+    case 25: return launch_turns<BITS, 1, 2, 8, EPI>(p, st);
+    case 26: return launch_turns<BITS, 1, 2, 16, EPI>(p, st);
     default: return hipErrorInvalidValue;
   }
 }

@@ -466,7 +466,7 @@ def test_qgemm_tall_blocks_odd_depths(dev, bits, zmode):
     choice where it takes them (K >= 4096, more 128 x 64 blocks than CUs)
     against the 64 x 64 shape."""
     rng = np.random.default_rng(700 + bits)
-    nv = L.ifr_quant_gemm_variants()
+    tall, wide = 21, 22
 
     def run(N, K, Ms, check):
         zero = None if zmode == "codebook" else rng.uniform(0, (1 << bits) - 1, size=(N, K // 128))
@@ -487,9 +487,9 @@ def test_qgemm_tall_blocks_odd_depths(dev, bits, zmode):
 
     def vs_oracle(lin, dl, q, sc, args, out):
         ref = po.qgemm(q, sc[:, 0], lin)
-        for v in (nv - 2, nv - 1):
+        for v in (tall, wide):
             rc = L.ifr_quant_gemm_variant(dev.ctx, dl, *args, v)
-            if bits == 8 and v == nv - 1:
+            if bits == 8 and v == wide:
                 assert rc == ia.IFR_EDECLINE
                 continue
             ia.check(rc, f"variant {v}")
@@ -542,3 +542,43 @@ def test_pack_maps_at_small_batch_edges(dev, M, monkeypatch):
     spec = [(i, 50 + 7 * i, 0, i % 2) for i in range(dec)] + [(dec, 300 + p, 1, int(p == M - dec - 1)) for p in range(M - dec)]
     monkeypatch.setattr(sys.modules[__name__], "PACK_CASES", [([60 + 7 * i for i in range(dec)] + [900], spec)])
     test_pack_maps_match_restatement(dev, 0)
+
+
+@pytest.mark.parametrize("bits,zmode", [(2, "codebook"), (4, "codebook"), (8, "codebook"), (2, "general"),
+                                        (4, "general")])
+def test_qgemm_turns_edges(dev, bits, zmode):
+    """Split K in turns: fewer groups than waves, one turn, partial last turns
+    and more turns than are in flight, partial row blocks and column tiles,
+    output off 16-byte alignment, each shape against the oracle; the SwiGLU
+    pair against the 32 x 128 row blocks."""
+    rng = np.random.default_rng(800 + bits)
+    for N, K, Ms in ((48, 128, (1, 33)), (80, 1024, (16, 65)), (32, 4224, (1, 17)), (48, 5248, (31, 64))):
+        zero = None if zmode == "codebook" else rng.uniform(0, (1 << bits) - 1, size=(N, K // 128))
+        lin, gate, up = (ia.make_linear(N, K, bits, rng, zero=zero) for _ in range(3))
+        dl, dp = C.c_void_p(), C.c_void_p()
+        ia.check(L.ifr_linear_upload(dev.ctx, C.byref(lin.struct), C.byref(dl)), "upload")
+        ia.check(L.ifr_linear_upload_pair(dev.ctx, C.byref(gate.struct), C.byref(up.struct), C.byref(dp)), "pair")
+        try:
+            for M in Ms:
+                q, sc, g = po.act_quant(rng.standard_normal((M, K), dtype=np.float32))
+                qd, sd, gd = dev.upload(ia.atile(q)), dev.upload(sc[:, 0].copy()), dev.upload(g)
+                od = dev.alloc(M * N * 2 + 16)
+                od2 = C.c_void_p(od.p.value + 2)
+                ref = po.qgemm(q, sc[:, 0], lin)
+                ia.check(L.ifr_quant_gemm_variant(dev.ctx, dp, qd.p, sd.p, gd.p, M, od.p, 5), "pair, row blocks")
+                pref = dev.download(od, np.uint16, (M, N))
+                for v in (23, 24, 25, 26):
+                    announce(f"turns variant {v} bits={bits} {zmode} N={N} K={K} M={M}")
+                    args = (qd.p, sd.p, gd.p, M)
+                    ia.check(L.ifr_quant_gemm_variant(dev.ctx, dl, *args, od.p, v), f"variant {v}")
+                    assert np.array_equal(dev.download(od, np.uint16, (M, N)), ref), (v, N, K, M)
+                    ia.check(L.ifr_quant_gemm_variant(dev.ctx, dl, *args, od2, v), f"unaligned {v}")
+                    raw = dev.download(od, np.uint16, (M * N + 8,))
+                    assert np.array_equal(raw[1:1 + M * N].reshape(M, N), ref), ("unaligned", v)
+                    ia.check(L.ifr_quant_gemm_variant(dev.ctx, dp, *args, od.p, v), f"pair {v}")
+                    assert np.array_equal(dev.download(od, np.uint16, (M, N)), pref), ("pair", v, N, K, M)
+                for b in (qd, sd, gd, od):
+                    b.free()
+        finally:
+            L.ifr_linear_free(dev.ctx, dl)
+            L.ifr_linear_free(dev.ctx, dp)
