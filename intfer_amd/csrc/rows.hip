@@ -326,16 +326,20 @@ __global__ __launch_bounds__(512) void row_quant1024_kernel(RowQuantArgs a) {
 // ---- any K (a multiple of 256, up to 8192): the row in registers -----------
 //
 // The row splits into the power-of-two head [0, P) the FWHT rotates
-// (blockdiag(H_P, I), spinquant.cpp:586-604) and the tail [P, K).  Thread t
-// holds the E = P / 256 contiguous head elements [E t, E t + E) and the
-// ET = (K - P) / 256 contiguous tail elements [P + ET t, +ET).  FWHT stages
+// (blockdiag(H_P, I), spinquant.cpp:586-604) and the tail [P, K).  Thread t of
+// T holds the E = P / T contiguous head elements [E t, E t + E) and the
+// ET = (K - P) / T contiguous tail elements [P + ET t, +ET).  FWHT stages
 // in the reference order: half < E inside the thread, half = E .. 32 E across
-// the lanes of a wave (partner lane ^ half / E), the last two (half = P / 4,
-// P / 2, across the four waves) through one LDS exchange, as fwht1024 does.
-// Every output is formed by the same adds on the same operands as the
-// sequential loop, and the RMS sum runs the reference's eight sequential
-// chains over the LDS copy of the row, so the result is bit-identical to the
-// LDS kernel it replaces.
+// the lanes of a wave (partner lane ^ half / E), the rest across the waves,
+// two stages per LDS exchange, as fwht1024 does.  Every output is formed by
+// the same adds on the same operands as the sequential loop, and the RMS sum
+// runs the reference's eight sequential chains over the LDS copy of the row,
+// so the result is bit-identical to the LDS kernel it replaces.
+// Bound by its chain of exchanges and the RMS chains (K / 8 dependent fused
+// steps), not by memory, so a wide row (K >= 4096) takes 1024 threads while
+// the rows leave CUs idle, and the chains read ahead: K 5120, normed and
+// rotated, one row 10.6 -> 9.1 us, 2160 rows 36.8 -> 35.7 (of which 17.3 without
+// norm and rotation).
 template <int M, int E>
 __device__ __forceinline__ void bfly_lanes(float (&v)[E]) {
 #pragma unroll
@@ -347,9 +351,9 @@ __device__ __forceinline__ void bfly_lanes(float (&v)[E]) {
 // instead of a few.
 __device__ __forceinline__ int pad32(int i) { return i + (i >> 5); }
 
-template <int E>
+template <int E, int T>
 __device__ void fwht_regs(float (&v)[E], float* xs) {
-  constexpr int P = 256 * E;
+  constexpr int P = T * E;
 #pragma unroll
   for (int half = 1; half < E; half <<= 1)
 #pragma unroll
@@ -365,20 +369,23 @@ __device__ void fwht_regs(float (&v)[E], float* xs) {
   bfly_lanes<8>(v);
   bfly_lanes<16>(v);
   bfly_lanes<32>(v);
-  __syncthreads();
-#pragma unroll
-  for (int e = 0; e < E; ++e) xs[pad32(E * threadIdx.x + e)] = v[e];
-  __syncthreads();
-  const int q = threadIdx.x >> 6;  // quarter of the P head elements
   const float inv = 1.0f / sqrtf((float)P);
 #pragma unroll
-  for (int e = 0; e < E; ++e) {
-    const int base = (E * threadIdx.x + e) & (P / 4 - 1);
-    const float a0 = xs[pad32(base)], a1 = xs[pad32(base + P / 4)], a2 = xs[pad32(base + P / 2)],
-                a3 = xs[pad32(base + 3 * P / 4)];
-    const float b0 = a0 + a1, b1 = a0 - a1, b2 = a2 + a3, b3 = a2 - a3;
-    const float c = q == 0 ? b0 + b2 : q == 1 ? b1 + b3 : q == 2 ? b0 - b2 : b1 - b3;
-    v[e] = c * inv;
+  for (int st = 64 * E; st < P; st *= 4) {  // stages half = st, 2 st
+    __syncthreads();
+#pragma unroll
+    for (int e = 0; e < E; ++e) xs[pad32(E * threadIdx.x + e)] = v[e];
+    __syncthreads();
+    const int q = (int)(threadIdx.x * E / st) & 3;  // quarter of the 4 st elements (wave-uniform)
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+      const int base = (E * threadIdx.x + e) & ~(3 * st);
+      const float a0 = xs[pad32(base)], a1 = xs[pad32(base + st)], a2 = xs[pad32(base + 2 * st)],
+                  a3 = xs[pad32(base + 3 * st)];
+      const float b0 = a0 + a1, b1 = a0 - a1, b2 = a2 + a3, b3 = a2 - a3;
+      const float c = q == 0 ? b0 + b2 : q == 1 ? b1 + b3 : q == 2 ? b0 - b2 : b1 - b3;
+      v[e] = 4 * st == P ? c * inv : c;
+    }
   }
 }
 
@@ -459,13 +466,13 @@ __device__ __forceinline__ void store_codes(int8_t* q, int m, int k0, int K, con
   }
 }
 
-template <int E>
-__global__ __launch_bounds__(256) void row_quant_wide(RowQuantArgs a) {
+template <int E, int T>
+__global__ __launch_bounds__(T) void row_quant_wide(RowQuantArgs a) {
   // the padded FWHT exchange (P + P / 32) or the chain-major row (K + 32)
   __shared__ __attribute__((aligned(16))) float xs[8192 + 256];
-  __shared__ float red[16];
-  constexpr int P = 256 * E;
-  const int K = a.K, ET = (K - P) / 256;
+  constexpr int P = T * E, NW = T / 64;
+  __shared__ float red[8 + NW];
+  const int K = a.K, ET = (K - P) / T;
   const int m = blockIdx.x, t = threadIdx.x, lane = t & 63;
   const int src = a.rowmap ? a.rowmap[m] : m;
   const size_t h0 = (size_t)src * K + (size_t)E * t, t0 = (size_t)src * K + P + (size_t)ET * t;
@@ -487,7 +494,7 @@ __global__ __launch_bounds__(256) void row_quant_wide(RowQuantArgs a) {
     ld_f32<E>(a.resid + t0, rw, ET);
     ld_f16<E>(a.y + h0, v, E);
     ld_f16<E>(a.y + t0, w, ET);
-    if (a.rot_y) fwht_regs<E>(v, xs);
+    if (a.rot_y) fwht_regs<E, T>(v, xs);
 #pragma unroll
     for (int e = 0; e < E; ++e) {
       v[e] = rv[e] + v[e];
@@ -518,10 +525,14 @@ __global__ __launch_bounds__(256) void row_quant_wide(RowQuantArgs a) {
     if (t < 8) {
       float acc = 0.0f;
       const float4* xc = reinterpret_cast<const float4*>(xs + t * CS);
-      for (int n4 = 0; n4 < K / 32; n4 += 8) {
-        float4 x8[8];
+      // the next eight float4 are read while these eight are summed
+      float4 x8[8], y8[8];
 #pragma unroll
-        for (int i = 0; i < 8; ++i) x8[i] = xc[n4 + i];
+      for (int i = 0; i < 8; ++i) x8[i] = xc[i];
+      for (int n4 = 0; n4 < K / 32; n4 += 8) {
+        const int nn = min(n4 + 8, K / 32 - 8);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) y8[i] = xc[nn + i];
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
           acc = fmaf(x8[i].x, x8[i].x, acc);
@@ -529,6 +540,8 @@ __global__ __launch_bounds__(256) void row_quant_wide(RowQuantArgs a) {
           acc = fmaf(x8[i].z, x8[i].z, acc);
           acc = fmaf(x8[i].w, x8[i].w, acc);
         }
+#pragma unroll
+        for (int i = 0; i < 8; ++i) x8[i] = y8[i];
       }
       red[t] = acc;
     }
@@ -545,7 +558,7 @@ __global__ __launch_bounds__(256) void row_quant_wide(RowQuantArgs a) {
       if (e < ET) w[e] = (w[e] * f) * (1.0f + nw[e]);
     }
   }
-  if (a.rotate) fwht_regs<E>(v, xs);
+  if (a.rotate) fwht_regs<E, T>(v, xs);
   // quantization: per row (ga 0) or per 64-wide slice (ga 64)
   float sh_ = 0.0f, st_ = 0.0f;  // scale of the head / tail element slices
   float ih = 0.0f, it = 0.0f;
@@ -560,7 +573,9 @@ __global__ __launch_bounds__(256) void row_quant_wide(RowQuantArgs a) {
     __syncthreads();
     if (lane == 0) red[8 + (t >> 6)] = mx;
     __syncthreads();
-    mx = fmaxf(1e-6f, fmaxf(fmaxf(red[8], red[9]), fmaxf(red[10], red[11])));
+#pragma unroll
+    for (int i = 0; i < NW; ++i) mx = fmaxf(mx, red[8 + i]);
+    mx = fmaxf(1e-6f, mx);
     sh_ = st_ = mx / 127.0f;
     ih = it = 1.0f / sh_;
     if (t == 0) a.qscale[m] = sh_;
@@ -608,7 +623,7 @@ __global__ __launch_bounds__(256) void row_quant_wide(RowQuantArgs a) {
     int* sred = reinterpret_cast<int*>(xs);
     if (lane == 0) {  // per-wave sums, for groups of 128 lanes (E or ET = 1)
       sred[t >> 6] = Sh;
-      sred[8 + (t >> 6)] = St;
+      sred[NW + (t >> 6)] = St;
     }
     __syncthreads();
     if ((E * t) % 128 == 0)
@@ -616,7 +631,7 @@ __global__ __launch_bounds__(256) void row_quant_wide(RowQuantArgs a) {
           (float)(128 / E > 64 ? sred[t >> 6] + sred[(t >> 6) + 1] : Sh);
     if (ET > 0 && (ET * t) % 128 == 0)
       a.gsum[(size_t)m * (K / 128) + (P + ET * t) / 128] =
-          (float)(128 / ET > 64 ? sred[8 + (t >> 6)] + sred[8 + (t >> 6) + 1] : St);
+          (float)(128 / ET > 64 ? sred[NW + (t >> 6)] + sred[NW + (t >> 6) + 1] : St);
   }
 }
 
@@ -1228,13 +1243,23 @@ hipError_t launch_row_quant(const RowQuantArgs& a, hipStream_t st) {
     while (2 * P <= a.K) P *= 2;
     const int et = (a.K - P) / 256;
     if (a.K % 256 == 0 && (et & (et - 1)) == 0) {
+      // 1024 threads a row while every row has a CU to itself (K 5120, M = 256:
+      // 11.8 -> 11.0 us; two rows a CU lose: M = 537 16.1 against 21.0)
+      const bool wide = a.M <= 256 && et % 4 == 0;
+      const dim3 grid(a.M);
       switch (P / 256) {
-        case 1: hipLaunchKernelGGL(row_quant_wide<1>, dim3(a.M), dim3(256), 0, st, a); return hipGetLastError();
-        case 2: hipLaunchKernelGGL(row_quant_wide<2>, dim3(a.M), dim3(256), 0, st, a); return hipGetLastError();
-        case 4: hipLaunchKernelGGL(row_quant_wide<4>, dim3(a.M), dim3(256), 0, st, a); return hipGetLastError();
-        case 8: hipLaunchKernelGGL(row_quant_wide<8>, dim3(a.M), dim3(256), 0, st, a); return hipGetLastError();
-        case 16: hipLaunchKernelGGL(row_quant_wide<16>, dim3(a.M), dim3(256), 0, st, a); return hipGetLastError();
-        case 32: hipLaunchKernelGGL(row_quant_wide<32>, dim3(a.M), dim3(256), 0, st, a); return hipGetLastError();
+        case 1: hipLaunchKernelGGL((row_quant_wide<1, 256>), grid, dim3(256), 0, st, a); return hipGetLastError();
+        case 2: hipLaunchKernelGGL((row_quant_wide<2, 256>), grid, dim3(256), 0, st, a); return hipGetLastError();
+        case 4: hipLaunchKernelGGL((row_quant_wide<4, 256>), grid, dim3(256), 0, st, a); return hipGetLastError();
+        case 8: hipLaunchKernelGGL((row_quant_wide<8, 256>), grid, dim3(256), 0, st, a); return hipGetLastError();
+        case 16:
+          if (wide) hipLaunchKernelGGL((row_quant_wide<4, 1024>), grid, dim3(1024), 0, st, a);
+          else hipLaunchKernelGGL((row_quant_wide<16, 256>), grid, dim3(256), 0, st, a);
+          return hipGetLastError();
+        case 32:
+          if (wide) hipLaunchKernelGGL((row_quant_wide<8, 1024>), grid, dim3(1024), 0, st, a);
+          else hipLaunchKernelGGL((row_quant_wide<32, 256>), grid, dim3(256), 0, st, a);
+          return hipGetLastError();
         default: break;
       }
     }

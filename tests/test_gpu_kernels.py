@@ -582,3 +582,28 @@ def test_qgemm_turns_edges(dev, bits, zmode):
         finally:
             L.ifr_linear_free(dev.ctx, dl)
             L.ifr_linear_free(dev.ctx, dp)
+
+
+@pytest.mark.parametrize("K,norm,rot,rnd,ga", [(4096, 1, 1, 0, 0), (5120, 1, 1, 0, 0), (5120, 1, 1, 1, 64),
+                                               (6144, 1, 1, 0, 0), (8192, 1, 1, 0, 64), (4352, 1, 1, 0, 0)])
+def test_act_quant_wide_rows_few_and_many(dev, K, norm, rot, rnd, ga):
+    """Rows of 4096 columns and more on both sides of the 256 rows up to which
+    a row takes 1024 threads (K = 4352: never, its tail does not divide), bit
+    for bit against the oracle."""
+    rng = np.random.default_rng(K + ga)
+    w = rng.normal(0, 0.1, size=K).astype(np.float32)
+    wd = dev.upload(w)
+    for M in (1, 256, 257):
+        x = (rng.standard_normal((M, K), dtype=np.float32) * 2.5).astype(np.float32)
+        q, s, g = po.act_quant(x, norm_w=w if norm else None, rotate=rot, round=rnd, ga=ga)
+        ns, Mp = K // ga if ga else 1, (M + 15) // 16 * 16
+        xd, qd, sd, gd = dev.upload(x), dev.alloc(Mp * K), dev.alloc(M * ns * 4), dev.alloc(M * (K // 128) * 4)
+        announce(f"act_quant K={K} M={M} ga={ga}")
+        ia.check(L.ifr_act_quant(dev.ctx, xd.p, M, K, wd.p if norm else None, C.c_float(1e-6), rot, rnd, ga, qd.p,
+                                 sd.p, gd.p), "ifr_act_quant")
+        assert np.array_equal(ia.untile(dev.download(qd, np.int8, (Mp * K,)), M, K), q), M
+        assert np.array_equal(dev.download(sd, np.float32, (M, ns)).view(np.uint32), s.view(np.uint32)), M
+        assert np.array_equal(dev.download(gd, np.float32, (M, K // 128)), g), M
+        for b in (xd, qd, sd, gd):
+            b.free()
+    wd.free()
