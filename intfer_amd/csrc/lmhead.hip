@@ -60,14 +60,26 @@ __global__ __launch_bounds__(256) void lmhead_kernel(LmP p) {
   for (int i = 0; i < WM; ++i)
 #pragma unroll
     for (int j = 0; j < kWN; ++j) acc[i][j] = (v4f){0.f, 0.f, 0.f, 0.f};
-  for (int s = 0; s < p.nsteps; ++s) {
-    v4i A[WM], B[kWN];
-#pragma unroll
-    for (int i = 0; i < WM; ++i) A[i] = *reinterpret_cast<const v4i*>(arow[i] + 1024 * s);
+  // R K steps of the weight stream in flight per wave beside the A rows of two
+  // (L2).  One step at a time reaches the stream's rate while many waves share a
+  // SIMD (32 rows with the argmax reduce: 38.7 us, with 4 steps 47.8); the
+  // 64-row block holds fewer and needs them: 64 rows 76.3 -> 64.6 us, of which
+  // the reduce is 5.
+  constexpr int R = WM == 4 ? 4 : 1;
+  v4i Bq[R][kWN];
+  auto load_b = [&](v4i (&B)[kWN], int s) {
+    s = min(s, p.nsteps - 1);
 #pragma unroll
     for (int j = 0; j < kWN; ++j)
       B[j] = __builtin_nontemporal_load(reinterpret_cast<const v4i*>(p.w) +
                                         ((size_t)tl[j] * p.nsteps + s) * 64 + lane);
+  };
+  auto load_a = [&](v4i (&A)[WM], int s) {
+    s = min(s, p.nsteps - 1);
+#pragma unroll
+    for (int i = 0; i < WM; ++i) A[i] = *reinterpret_cast<const v4i*>(arow[i] + 1024 * s);
+  };
+  auto mac = [&](const v4i (&A)[WM], const v4i (&B)[kWN], int s) {
 #pragma unroll
     for (int i = 0; i < WM; ++i) {
       float asr[4];
@@ -78,6 +90,28 @@ __global__ __launch_bounds__(256) void lmhead_kernel(LmP p) {
         const v4i T = __builtin_amdgcn_mfma_i32_16x16x64_i8(A[i], B[j], (v4i){0, 0, 0, 0}, 0, 0, 0);
 #pragma unroll
         for (int r = 0; r < 4; ++r) acc[i][j][r] = fmaf((float)T[r], asr[r], acc[i][j][r]);
+      }
+    }
+  };
+  if constexpr (R == 1) {
+    for (int s = 0; s < p.nsteps; ++s) {
+      v4i A[WM];
+      load_a(A, s);
+      load_b(Bq[0], s);
+      mac(A, Bq[0], s);
+    }
+  } else {
+    v4i Aq[2][WM];
+    load_a(Aq[0], 0);
+#pragma unroll
+    for (int d = 0; d < R; ++d) load_b(Bq[d], d);
+    for (int s0 = 0; s0 < p.nsteps; s0 += R) {
+#pragma unroll
+      for (int d = 0; d < R; ++d) {
+        if (s0 + d >= p.nsteps) break;
+        load_a(Aq[(d + 1) & 1], s0 + d + 1);
+        mac(Aq[d & 1], Bq[d], s0 + d);
+        load_b(Bq[d], s0 + d + R);
       }
     }
   }
@@ -115,34 +149,53 @@ __global__ __launch_bounds__(256) void lmhead_kernel(LmP p) {
     }
 }
 
-// Reduce the per-wave (value, index) partials of each row in part order.
-__global__ __launch_bounds__(256) void argmax_final_kernel(const float* pv, const int32_t* pi,
-                                                           int nparts, int W, int32_t* best) {
-  const int row = blockIdx.x;
+// Reduce the per-wave (value, index) partials of each row.  Bound by the
+// latency of reading them: 1024 threads, four partials of each in flight (V =
+// 151936, 4748 partials a row: lm_head and reduce of 8 rows 38.0 -> 33.4 us
+// against 256 threads with one in flight).
+__global__ __launch_bounds__(1024) void argmax_final_kernel(const float* pv, const int32_t* pi,
+                                                            int nparts, int W, int32_t* best) {
+  const int row = blockIdx.x, lane = threadIdx.x & 63;
+  pv += (size_t)row * nparts;
+  pi += (size_t)row * nparts;
   float bv = -INFINITY;
   int bi = 0x7fffffff;
-  for (int q = threadIdx.x; q < nparts; q += blockDim.x) {
-    const float v = pv[(size_t)row * nparts + q];
-    const int i = pi[(size_t)row * nparts + q];
-    if (better(v, i, bv, bi)) { bv = v; bi = i; }
-  }
-  __shared__ float sv[256];
-  __shared__ int si[256];
-  sv[threadIdx.x] = bv;
-  si[threadIdx.x] = bi;
-  __syncthreads();
-  for (int s = 128; s > 0; s >>= 1) {
-    if ((int)threadIdx.x < s) {
-      if (better(sv[threadIdx.x + s], si[threadIdx.x + s], sv[threadIdx.x], si[threadIdx.x])) {
-        sv[threadIdx.x] = sv[threadIdx.x + s];
-        si[threadIdx.x] = si[threadIdx.x + s];
-      }
+  for (int q0 = threadIdx.x; q0 < nparts; q0 += 4 * 1024) {
+    float v[4];
+    int i[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {  // past the end: this thread's first partial again
+      const int q = q0 + 1024 * k < nparts ? q0 + 1024 * k : q0;
+      v[k] = pv[q];
+      i[k] = pi[q];
     }
-    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+      if (better(v[k], i[k], bv, bi)) { bv = v[k]; bi = i[k]; }
   }
+  auto wave_best = [&] {
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const float ov = __shfl_xor(bv, o, 64);
+      const int oi = __shfl_xor(bi, o, 64);
+      if (better(ov, oi, bv, bi)) { bv = ov; bi = oi; }
+    }
+  };
+  __shared__ float sv[16];
+  __shared__ int si[16];
+  wave_best();
+  if (lane == 0) {
+    sv[threadIdx.x >> 6] = bv;
+    si[threadIdx.x >> 6] = bi;
+  }
+  __syncthreads();
+  if (threadIdx.x >= 64) return;  // (after the only barrier)
+  bv = sv[lane & 15];
+  bi = si[lane & 15];
+  wave_best();
   // The reference starts from -1e30 with strict '>': a row whose logits are
   // all <= -1e30 reports -1.
-  if (threadIdx.x == 0) best[row] = (sv[0] > -1e30f) ? si[0] : -1;
+  if (threadIdx.x == 0) best[row] = (bv > -1e30f) ? bi : -1;
 }
 
 template <int WM>
@@ -174,7 +227,7 @@ hipError_t launch_lmhead(LmHeadArgs& a, hipStream_t st) {
   else if (a.W <= 64) e = launch_wm<4>(p, a.nparts, 1, st);
   else e = launch_wm<4>(p, a.nparts, (a.W + 63) / 64, st);
   if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(argmax_final_kernel, dim3(a.W), dim3(256), 0, st, a.part_val, a.part_idx,
+  hipLaunchKernelGGL(argmax_final_kernel, dim3(a.W), dim3(1024), 0, st, a.part_val, a.part_idx,
                      a.nparts, a.W, a.best);
   return hipGetLastError();
 }
