@@ -607,3 +607,30 @@ def test_act_quant_wide_rows_few_and_many(dev, K, norm, rot, rnd, ga):
         for b in (xd, qd, sd, gd):
             b.free()
     wd.free()
+
+
+@pytest.mark.parametrize("hidden,vocab", [(256, 528), (768, 140016)])
+def test_lm_head_row_blocks(dev, hidden, vocab):
+    """The lm_head where its row blocks end (64 rows: several K steps of
+    weights in flight, 4 steps and 12 here), on more and fewer partials a row
+    than the argmax reduce reads in one pass.  Sequences of one token, whose
+    attention is exact: tokens and logit rows bit for bit, up to a rare ulp of
+    SwiGLU's device expf (test_single_token_sequences_bit_exact)."""
+    cfg = ia.default_cfg(layers=1, hidden=hidden, inter=256, n_heads=2, n_kv=1, vocab=vocab)
+    m = ia.SynthModel(cfg, seed=21)
+    eng = ia.Engine(dev, m, max_seqs=80, max_seq_tokens=64, max_rows=80)
+    ora = po.OracleEngine(m, kv_int8=0, mode=0, max_seqs=80)
+    for W in (32, 33, 64, 65):
+        se, so = [eng.seq_open() for _ in range(W)], [ora.seq_open() for _ in range(W)]
+        toks = [(7 + 131 * i) % vocab for i in range(W)]
+        announce(f"lm_head hidden={hidden} vocab={vocab} rows={W}")
+        be, lg = eng.forward([(s, 0, t, ia.ROW_DECODE, 1) for s, t in zip(se, toks)], logits=True)
+        bo, lo = ora.forward([(s, 0, t, ia.ROW_DECODE, 1) for s, t in zip(so, toks)], logits=True)
+        exact = sum(np.array_equal(lg[r].view(np.uint32), lo[r].view(np.uint32)) for r in range(W))
+        assert np.array_equal(be, lg.argmax(1)) and exact >= W - 1 - W // 6, (W, exact)
+        assert np.abs(lg - lo).max() < 2e-2 * lo.std(), W
+        for s in se:
+            eng.seq_close(s)
+        for s in so:
+            ora.seq_close(s)
+    m.close()
