@@ -1355,6 +1355,12 @@ __global__ __launch_bounds__(64 * NWV) void qgemm_turns(KParams p) {
 #pragma unroll
   for (int i = 0; i < WM; ++i) at[i] = (uint32_t)(min((bm0 >> 4) + i, (p.M - 1) >> 4) * p.nsteps);
 
+  // One row tile: the lanes of rows past M read row M - 1 (outputs never
+  // stored), so a 1 KB A tile costs its real rows' lines only; every block reads
+  // the whole A, at 16 padded rows more bytes than its INT2 codes (down 17408 ->
+  // 5120, 2 to 8 rows: 12.4 -> 11.7 us; 9 rows and more read the same lines).
+  const int alane = WM == 1 ? 16 * lgrp + min(lrow, p.M - 1 - bm0) : lane;
+
   uint32_t Bw[RB][2][WN][BITS / 2];
   v4i A[RA][2][WM];
   auto fetch_b = [&](uint32_t (&B)[2][WN][BITS / 2], int t) {
@@ -1371,7 +1377,7 @@ __global__ __launch_bounds__(64 * NWV) void qgemm_turns(KParams p) {
     for (int h = 0; h < 2; ++h)
 #pragma unroll
       for (int i = 0; i < WM; ++i)
-        a[h][i] = reinterpret_cast<const v4i*>(p.a + (size_t)(at[i] + 2 * g + h) * 1024)[lane];
+        a[h][i] = reinterpret_cast<const v4i*>(p.a + (size_t)(at[i] + 2 * g + h) * 1024)[alane];
   };
   // a turn's S and scale | zero pairs, one value of each per thread
   const int sr = threadIdx.x / NWV, sg = threadIdx.x % NWV;
