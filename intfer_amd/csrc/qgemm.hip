@@ -1965,15 +1965,20 @@ hipError_t launch_bits(const KParams& p, int variant, hipStream_t st) {
     // to M = 4 and one above, one tile pair of 8 waves for the SwiGLU pair; its
     // fold grows with the rows and its parked d with rows and depth, so split K
     // in turns takes over above 8 rows (M = 16, us: QKV 7.3 -> 6.7, O 7.2 ->
-    // 6.6, gate/up 27.5 -> 21.8, INT4 38.0 -> 28.8) and on the deep down
-    // projection (16 waves) above one row, INT4 above 4 (M = 4 13.4 -> 12.5, 16
-    // 20.3 -> 12.7, M = 1 11.7 against 12.4; INT4 M = 8 20.4 -> 16.8).  A shape
-    // a variant cannot hold (registers or LDS for wider codes) falls back to
-    // the next one, then to the choice above.
+    // 6.6, gate/up 27.5 -> 21.8, INT4 38.0 -> 28.8), INT4 above 4 for the plain
+    // projections (M = 8: QKV 7.9 -> 7.6, O 7.8 -> 7.4; M = 4 7.15 against 7.6),
+    // and on the deep down projection above one row with 16 waves (M = 4 13.4 ->
+    // 11.7, 16 20.3 -> 12.5, M = 1 11.5 against 11.7; 8 waves 14.5), INT4 above 3
+    // with 8 waves, whose codes fit the registers (M = 4 16.7 -> 16.0, 16 waves
+    // 16.5; M = 8 20.4 -> 16.0; M = 2 15.4 against 16.0).  16-column blocks (320
+    // workgroups for down) lose: 14.0 with 8 waves, 17.4 with 16.  A shape a
+    // variant cannot hold (registers or LDS for wider codes) falls back to the
+    // next one, then to the choice above.
     if (p.K >= 4096 && p.M <= 16) {
       hipError_t e = hipErrorInvalidValue;
       const bool deep = EPI == 0 && p.ng >= 96;
-      if (deep ? p.M > (BITS == 2 ? 1 : 4) : p.M > 8) e = launch_bits<BITS, EPI>(p, deep ? 26 : 25, st);
+      const int turns_above = deep ? (BITS == 2 ? 1 : BITS == 4 ? 3 : 4) : BITS == 4 && EPI == 0 ? 4 : 8;
+      if (p.M > turns_above) e = launch_bits<BITS, EPI>(p, deep && BITS != 4 ? 26 : 25, st);
       if (e != hipErrorInvalidValue) return e;
       if (EPI == 1) {
         e = launch_bits<BITS, EPI>(p, 14, st);

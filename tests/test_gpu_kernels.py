@@ -634,3 +634,22 @@ def test_lm_head_row_blocks(dev, hidden, vocab):
         for s in so:
             ora.seq_close(s)
     m.close()
+
+
+@pytest.mark.parametrize("bits", [2, 4, 8])
+def test_qgemm_default_few_deep_rows(dev, bits):
+    """The default choice between the weight stream and split K in turns, on
+    both sides of each of its row counts, bit for bit against the oracle."""
+    rng = np.random.default_rng(900 + bits)
+    for N, K in ((48, 4096), (48, 5120), (32, 12288)):
+        lin, dl = ia.make_linear(N, K, bits, rng), C.c_void_p()
+        ia.check(L.ifr_linear_upload(dev.ctx, C.byref(lin.struct), C.byref(dl)), "upload")
+        for M in (1, 2, 3, 4, 5, 8, 9, 16, 17):
+            q, sc, g = po.act_quant(rng.standard_normal((M, K), dtype=np.float32))
+            qd, sd, gd, od = dev.upload(ia.atile(q)), dev.upload(sc[:, 0].copy()), dev.upload(g), dev.alloc(M * N * 2)
+            announce(f"few deep rows bits={bits} N={N} K={K} M={M}")
+            ia.check(L.ifr_quant_gemm(dev.ctx, dl, qd.p, sd.p, gd.p, M, od.p, None), "default")
+            assert np.array_equal(dev.download(od, np.uint16, (M, N)), po.qgemm(q, sc[:, 0], lin)), (N, K, M)
+            for b in (qd, sd, gd, od):
+                b.free()
+        L.ifr_linear_free(dev.ctx, dl)
