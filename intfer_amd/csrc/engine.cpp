@@ -526,8 +526,8 @@ int prep_sub(ifr_ctx* c, const ifr_row* rows, SubBatch& sb) {
 // The rows as the pack kernel reads them: into the lane's pinned buffer, and
 // from there read in place up to kPackSmallRows rows (a copy is a launch of its
 // own ahead of the pack kernel, 3 us longer than the read over the bus that
-// replaces it), else through its device copy.  The buffer is free: the lane's last
-// batch was waited for.
+// replaces it), else through its device copy.  The buffer is free: every call
+// that queues its reader waits for it, also on its error returns (Drain).
 int stage_rows(Lane& L, const ifr_row* r, int M, hipStream_t st, const int32_t** src) {
   std::memcpy(L.rows_h, r, (size_t)M * sizeof(ifr_row));
   *src = L.rows_h;
@@ -537,6 +537,19 @@ int stage_rows(Lane& L, const ifr_row* r, int M, hipStream_t st, const int32_t**
   }
   return IFR_OK;
 }
+
+// Waits for a call's streams where it returns early: what it queued reads the
+// pinned rows that the next call overwrites (and, in ifr_attention_noalloc, the
+// device's scratch).  The way to IFR_OK disarms it after its own wait.
+struct Drain {
+  const ifr_ctx* c;
+  bool armed = true;
+  explicit Drain(const ifr_ctx* c_) : c(c_) {}
+  ~Drain() {
+    if (!armed) return;
+    for (const Lane& L : c->lane) hipStreamSynchronize(L.st);
+  }
+};
 
 // Rows up; the pack kernel writes the packing maps and the token column.
 int launch_head(ifr_ctx* c, const ifr_row* rows, const SubBatch& sb) {
@@ -1477,6 +1490,7 @@ int ifr_forward(ifr_ctx* c, const ifr_row* rows, int32_t M, int32_t* best_out, f
     sbs.push_back(std::move(sb));
   }
   c->last_lanes = (int)sbs.size();
+  Drain drain(c);
   if (sbs.size() == 2) {
     HIPCHK(hipEventRecord(c->ev_bt, c->lane[0].st));
     HIPCHK(hipStreamWaitEvent(c->lane[1].st, c->ev_bt, 0));
@@ -1495,6 +1509,7 @@ int ifr_forward(ifr_ctx* c, const ifr_row* rows, int32_t M, int32_t* best_out, f
   }
   const auto t_sub = std::chrono::steady_clock::now();
   for (SubBatch& sb : sbs) HIPCHK(hipStreamSynchronize(c->lane[sb.lane].st));
+  drain.armed = false;
   const auto t_end = std::chrono::steady_clock::now();
   // host buckets (the reference engine's submit / waitblock profile,
   // engine.hpp:567-630), kept whether or not kernels are timed
@@ -1562,6 +1577,7 @@ int ifr_attention(ifr_ctx* c, int32_t layer, const ifr_row* rows, int32_t M, con
                                                 c->qb, &nchunked);
   c->last_slots = nslots;
   const int32_t* src = nullptr;
+  Drain drain(c);
   if (int r = stage_rows(c->lane[0], rows, M, c->st, &src)) return r;
   HIPCHK(ifrk::launch_pack(src, M, nkv, c->qb, split, c->lane[0].pk, c->st));
   HIPCHK(hipMemcpyAsync(c->lane[0].qbuf, q_h, (size_t)M * nq * hd * 2, hipMemcpyHostToDevice, c->st));
@@ -1588,6 +1604,7 @@ int ifr_attention(ifr_ctx* c, int32_t layer, const ifr_row* rows, int32_t M, con
   if (e == hipSuccess) e = hipStreamSynchronize(c->st);
   hipFree(out_d);
   HIPCHK(e);
+  drain.armed = false;
   if (c->timing) flush_timers(c);
   return IFR_OK;
 }
@@ -1635,6 +1652,7 @@ int ifr_attention_noalloc(ifr_ctx* c, int32_t layer, const ifr_row* rows, int32_
   // is read (the pack maps, each unit's partials, the combine outputs), so
   // nothing is cleared between calls
   const int32_t* src = rows_d;
+  Drain drain(c);  // (before the lock is given back)
   if (M <= c->maxM) {
     if (int r = stage_rows(c->lane[0], rows, M, c->st, &src)) return r;
   } else {  // more rows than the engine's own buffers hold
@@ -1652,6 +1670,7 @@ int ifr_attention_noalloc(ifr_ctx* c, int32_t layer, const ifr_row* rows, int32_
   HIPCHK(ifrk::launch_combine(cb, c->st));
   // the rows are read from host memory; return once out_d is written
   HIPCHK(hipStreamSynchronize(c->st));
+  drain.armed = false;
   return IFR_OK;
 }
 

@@ -11,6 +11,7 @@
 #include <cstdio>
 #include <cstdlib>
 #include <map>
+#include <set>
 #include <string>
 #include <vector>
 
@@ -101,6 +102,8 @@ struct Sched {
 
 Sched* g_s = nullptr;
 int g_err = hipSuccess;
+int g_launches = 0, g_fail_launch = 0, g_fail_malloc = 0;
+std::set<hipStream_t> g_queued;  // streams with work that nothing has waited for
 thread_local ThreadCtx g_host_ctx{};
 
 Sched& S() {
@@ -267,6 +270,8 @@ void emu_set_err(int e) {
   if (e != hipSuccess) g_err = e;
 }
 
+void note_queued(hipStream_t st) { g_queued.insert(st); }
+
 const unsigned char* wave_exchange(const void* mine, int bytes, int op) {
   Sched& s = S();
   if (s.current < 0) fail("cross-lane operation outside a kernel");
@@ -327,6 +332,8 @@ int launch_raw(KernelBody body, void* args, dim3 g, dim3 b, size_t shmem) {
     return hipErrorInvalidValue;
   }
   if (s.current >= 0) fail("kernel launch from inside a kernel");
+  ++g_launches;
+  if (g_fail_launch > 0 && --g_fail_launch == 0) return hipErrorOutOfMemory;
   s.body = body;
   s.args = args;
   s.dyn_bytes = shmem;
@@ -340,6 +347,14 @@ int launch_raw(KernelBody body, void* args, dim3 g, dim3 b, size_t shmem) {
 }
 
 }  // namespace emu
+
+// ---- failures on demand, for the tests of error returns: the k-th kernel
+// launch or hipMalloc from now fails (0: none); the launches so far; the
+// streams that hold work nothing has waited for
+extern "C" void emu_fail_launch(int k) { emu::g_fail_launch = k; }
+extern "C" void emu_fail_malloc(int k) { emu::g_fail_malloc = k; }
+extern "C" int emu_launches() { return emu::g_launches; }
+extern "C" int emu_unwaited() { return (int)emu::g_queued.size(); }
 
 // ---- builtins ------------------------------------------------------------------------
 
@@ -489,6 +504,7 @@ hipError_t hipGetDeviceProperties(hipDeviceProp_t* p, int) {
   return hipSuccess;
 }
 hipError_t hipMalloc(void** p, size_t n) {
+  if (emu::g_fail_malloc > 0 && --emu::g_fail_malloc == 0) return hipErrorOutOfMemory;
   // uninitialized device memory holds a recognizable pattern (0xCD bytes)
   void* q = std::malloc(n ? n : 1);
   if (!q) return hipErrorOutOfMemory;
@@ -514,7 +530,8 @@ hipError_t hipMemcpy(void* d, const void* s, size_t n, hipMemcpyKind) {
   if (n) std::memmove(d, s, n);
   return hipSuccess;
 }
-hipError_t hipMemcpyAsync(void* d, const void* s, size_t n, hipMemcpyKind k, hipStream_t) {
+hipError_t hipMemcpyAsync(void* d, const void* s, size_t n, hipMemcpyKind k, hipStream_t st) {
+  emu::note_queued(st);
   return hipMemcpy(d, s, n, k);
 }
 hipError_t hipMemset(void* d, int v, size_t n) {
@@ -531,8 +548,14 @@ hipError_t hipStreamDestroy(hipStream_t s) {
   delete reinterpret_cast<int*>(s);
   return hipSuccess;
 }
-hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
-hipError_t hipDeviceSynchronize() { return hipSuccess; }
+hipError_t hipStreamSynchronize(hipStream_t st) {
+  emu::g_queued.erase(st);
+  return hipSuccess;
+}
+hipError_t hipDeviceSynchronize() {
+  emu::g_queued.clear();
+  return hipSuccess;
+}
 hipError_t hipEventCreate(hipEvent_t* e) {
   *e = reinterpret_cast<hipEvent_t>(new double(0.0));
   return hipSuccess;

@@ -133,9 +133,11 @@ int launch(void (*k)(P...), dim3 g, dim3 b, size_t shmem, A&&... a) {
 #define blockDim (::emu::cur()->bdim)
 #define gridDim (::emu::cur()->gdim)
 
-#define hipLaunchKernelGGL(K, G, B, S, ST, ...) ((void)(ST), ::emu::emu_set_err(::emu::launch(K, dim3(G), dim3(B), (size_t)(S), ##__VA_ARGS__)))
+#define hipLaunchKernelGGL(K, G, B, S, ST, ...) \
+  (::emu::note_queued(ST), ::emu::emu_set_err(::emu::launch(K, dim3(G), dim3(B), (size_t)(S), ##__VA_ARGS__)))
 namespace emu {
 void emu_set_err(int e);
+void note_queued(hipStream_t st);  // work went onto st (until the stream is waited for)
 }
 
 inline void __syncthreads() { emu::block_barrier(); }

@@ -599,6 +599,63 @@ def forward_gated():
 
 
 @scenario
+def error_returns():
+    """A call that fails in the middle leaves nothing of it on the device's
+    streams: the pack kernel reads the call's rows in place from the engine's
+    pinned buffer, which the next call overwrites.  Every launch of the calls
+    that read it (one and two lanes), and ifr_attention's allocation, fails
+    once."""
+    import intfer_amd as ia
+    L = ia.lib()
+    dev = ia.Device(0)
+    model = ia.SynthModel(_small_cfg(ia, layers=1), seed=5, bits=2)
+    nq, hd = 4, 128
+    q = np.zeros((40, nq, hd), np.float16)
+    qd, od = dev.upload(q), dev.alloc(40 * nq * hd * 4)
+    for lanes in (1, 2):
+        eng = ia.Engine(dev, model, max_seqs=4, max_seq_tokens=256, pool_tokens=4 * 256, max_rows=64, lanes=lanes)
+        a, b = eng.seq_open(), eng.seq_open()
+        eng.forward([(a, p, 7 + p, ia.ROW_PREFILL, int(p == 19)) for p in range(20)])
+        rows = [(a, 10 + p, 0, ia.ROW_PREFILL, 0) for p in range(10)]
+        arr = ia.rows_array(rows)
+
+        def forward():
+            best = np.empty(41, np.int32)
+            batch = ia.rows_array([(a, 20, 5, ia.ROW_DECODE, 1)] + [(b, p, 9 + p, ia.ROW_PREFILL, 0) for p in range(40)])
+            rc = L.ifr_forward(dev.ctx, batch, 41, best.ctypes.data_as(C.POINTER(C.c_int32)), None)
+            if rc == 0:
+                eng.seq_truncate(a, 20)
+                eng.seq_truncate(b, 0)
+            return rc
+
+        def attention():
+            out = np.empty((10, nq * hd), np.float32)
+            return L.ifr_attention(dev.ctx, 0, arr, 10, q.ctypes.data_as(C.POINTER(C.c_uint16)),
+                                   out.ctypes.data_as(C.POINTER(C.c_float)))
+
+        def noalloc():
+            return L.ifr_attention_noalloc(dev.ctx, 0, arr, 10, qd.p, od.p)
+
+        for call in (forward, attention, noalloc):
+            n = L.emu_launches()
+            assert call() == 0, L.ifr_last_error()
+            n = L.emu_launches() - n
+            for k in range(1, n + 1):
+                L.emu_fail_launch(k)
+                assert call() < 0, (call.__name__, k)
+                assert L.emu_unwaited() == 0, (call.__name__, lanes, k)
+            assert call() == 0, L.ifr_last_error()
+            say(f"lanes={lanes} {call.__name__}: {n} failed launches, nothing left behind")
+        L.emu_fail_malloc(1)
+        assert attention() < 0 and L.emu_unwaited() == 0
+        del eng
+    qd.free()
+    od.free()
+    dev.close()
+    model.close()
+
+
+@scenario
 def prefix_copy():
     """ifr_seq_copy_prefix (the prefix cache's page copy) with fp16 and int8
     KV: a copied prefix plus the recomputed rest gives the same logits, bit

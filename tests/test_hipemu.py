@@ -35,7 +35,7 @@ def emu_lib():
 # waits for its own
 ORDER = ["gemm_stream", "gemm_stream_rows", "gemm_full", "forward_fused_qk", "prefix_copy", "gemm_small",
          "forward_gated", "noalloc_limits", "gemm_grouped", "gemm_f16", "gemm_ga", "attention_ragged_g5",
-         "forward_gqa5", "attention_ragged", "smoke", "act_quant", "intfer_load"]
+         "forward_gqa5", "attention_ragged", "smoke", "act_quant", "error_returns", "intfer_load"]
 
 
 @pytest.fixture(scope="module")
@@ -80,3 +80,7 @@ def test_fused_qk_epilogue_in_bounds_and_bit_identical(emu_runs):
 
 def test_attention_output_gate_in_bounds(emu_runs):
     assert emu_runs.result(["forward_gated"], timeout=1800) == 0
+
+
+def test_failed_call_leaves_nothing_queued(emu_runs):
+    assert emu_runs.result(["error_returns"], timeout=1800) == 0
