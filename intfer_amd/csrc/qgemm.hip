@@ -1882,6 +1882,104 @@ hipError_t launch_bits_qk(const KParams& p, int variant, hipStream_t st) {
   }
 }
 
+// The wide shapes (K >= 4096), M > 16: split K in turns (23, 24), 64 x 64 or
+// 128 x 64 blocks (3, 9), the tall blocks (21, 22) or `rows`, the row blocks of
+// launch_bits.  The lines were placed over K 4096 .. 17408, N 1024 .. 28672,
+// gate/up pairs of 6144 .. 57344, 2, 4 and 8 bits, M 17 .. 2160, so that no
+// point loses more than 6 % to `rows` with its weights coming from HBM (the
+// times below, us, where not said otherwise), or 9 % with them in the caches.
+template <int BITS>
+int wide_shape(const KParams& p, int rows) {
+  auto blocks = [&](long bm, long bn) { return ((p.M + bm - 1) / bm) * ((p.N + bn - 1) / bn); };
+  // Split K in turns while its 32 x 32 blocks are few: one per CU, at 2 bits
+  // two, or 2.5 where a row block walks 96 groups or more (N 5120, K 5120: M =
+  // 32 8.1 against 22.1, 96 11.8 against 21.7, 128 16.6 against 14.7 of 64 x
+  // 64; K 17408: 128 43.2 against 49.8, 160 54.1 against 49.8); INT4 and INT8
+  // hold one per CU, then 64 x 32 (K 17408, M = 64: 32.8 and 36.2 against 70.8
+  // and 76.7).  Up to 32 rows every 64-row block is half empty and 32 x 128
+  // blocks leave CUs idle, so further there: two per CU; at 2 bits three, four
+  // from 64 groups on (pair 2 x 14336, K 4096: 20.8 against 19.3 of 32 x 128,
+  // K 8192 29.8 against 33.9); and where 32 x 128 blocks need a second round of
+  // the CUs (pair 2 x 17408, K 5120: 27.8 against 30.0, INT4 38.4 against 40.1,
+  // INT8 52.8 against 51.5).
+  const long w = blocks(32, 32);
+  const bool few = w <= 512 || (BITS == 2 && w <= (p.ng >= 64 ? 1024 : 768)) ||
+                   (BITS != 8 && p.ng >= 40 && w > 1024 && w <= 1280);
+  if (w <= 256 || (BITS == 2 && w <= (p.ng >= 96 ? 640 : 512)) || (p.M <= 32 && few)) return 24;
+  if (BITS != 2 && blocks(64, 32) <= 256) return 23;
+  // 64 x 64 while one round of the CUs holds them, for their shorter groups
+  // (N 5120, K 5120, M = 128: 14.7 against 21.7).  The unpack of wider codes
+  // eats that: INT8 above 32 groups (K 8192, N 8192, M = 96: 38.8 against
+  // 34.0) only from M = 384, INT4 not at 64 .. 127 groups up to M = 128 (the
+  // same point: 29.2 against 27.8 from the caches).
+  if (blocks(64, 64) <= 256) {
+    const bool loses = BITS == 8 ? p.ng > 32 && p.M < 384 : BITS == 4 && p.ng >= 64 && p.ng < 128 && p.M <= 128;
+    return loses ? rows : 3;
+  }
+  // 128 x 64 the same way, unless 32 x 128 fits the round too (M = 160 pads to
+  // 256 rows: K 8192, N 6144 36.9 against 32.0); INT4 K 5120, N 7168, M = 160
+  // 28.5 against 36.7, INT2 K 7168 32.5 against 38.1, but K 5120, M = 256 27.1
+  // against 27.0 (from the caches 24.1 against 22.2).
+  if (blocks(128, 64) <= 256)
+    return blocks(32, 128) > 256 && (BITS != 2 || p.ng > 40 || p.M >= 1024) ? 9 : rows;
+  if (p.M <= 32) return rows;
+  // The tall blocks, whose time per CU is about 31, 36 and 48 us for 1, 2 and
+  // 3 of 64 x 128 and 48 and 59 us for 1 and 2 of 64 x 256, in these rounds
+  // (K 5120, M = 1024, N 5120: 48.2 and 59.5; N 7168: 73.7 and 59.3); not
+  // while `rows` fits the two workgroups a CU holds and the tall blocks start
+  // a round (K 4096, N 12288, M = 160: 28.7 against 23.7; the general fold and
+  // 32 groups at 2 bits, whose row blocks are cheap, three: N 5120, M = 512
+  // 29.3 against 29.7, from the caches 28.5 against 24.0).
+  const bool cheap = BITS == 2 && p.ng <= 32;
+  const long keep5 = BITS == 2 ? (cheap || !p.ff ? 768 : p.ng < 128 ? 512 : 0) : BITS == 4 ? (p.ng < 64 ? 512 : 0)
+               : p.ng <= 32 && p.M > 128 ? 512 : 0;
+  if (rows == 5 && blocks(32, 128) <= keep5) return rows;
+  if (rows == 6 && cheap && blocks(32, 256) <= 512) return rows;
+  if (rows != 5 && blocks(64, 128) <= 256 && (BITS == 2 || p.ng < 96)) return rows;
+  const long n21 = (blocks(64, 128) + 255) / 256, n22 = (blocks(64, 256) + 255) / 256;
+  const long t21 = 48 * (n21 / 3) + (n21 % 3 == 0 ? 0 : n21 % 3 == 1 ? 31 : 36);
+  const long t22 = 59 * (n22 / 2) + 48 * (n22 % 2);
+  return t22 < t21 ? 22 : 21;
+}
+
+// Split K in turns for M <= 16 on the wide shapes (8 waves: 25, 16 waves: 26),
+// 0 for the weight stream or the row blocks; placed as wide_shape's lines.
+// The plain stream's 16-column workgroups fill the CUs once up to N = 4096 and
+// take a second round beyond it, where turns' 32 columns do not (K 5120, M = 9,
+// us: N 4096 6.5 against the stream's 5.2, N 5120 6.6 against 6.9); the
+// stream's fold grows with the rows and its parked d with rows and depth.
+template <int BITS, int EPI>
+int decode_turns(const KParams& p) {
+  const long w = (p.N + 31) / 32;  // workgroups
+  if (EPI == 1) {
+    // Pairs above 8 rows, against 32 x 128 blocks, which need a second round
+    // of the CUs from w = 1024 on (2 x 17408, K 5120, M = 16: 22.0 against 27.7;
+    // INT4 2 x 14336, K 4096 21.0 against 20.7; INT8 2 x 25600 63.0 against 51.5).
+    if (p.M <= 8) return 0;
+    const long most = BITS == 2 ? 1280 : BITS == 4 ? 768 : 512;
+    return (BITS != 8 && p.ng > 40) || w <= most || (w > 1024 && w <= 1280) ? 25 : 0;
+  }
+  const bool two = p.N > 4096;
+  if (p.ng >= 96) {
+    // The deep down projection (K 17408, N 5120): INT2 with 16 waves above one
+    // row (M = 4 11.8 against 13.3, M = 8 11.9 against 16.9; N 4096, M = 8 11.7
+    // against 9.5); INT4 with 8, whose codes fit the registers (M = 4 16.0
+    // against 16.5, 16 waves 16.4), and INT8 above 4 rows (M = 8 21.6 against
+    // 24.7; 16 waves spill, 28.9).  Up to 4 rows the stream takes 32 columns too.
+    if (BITS == 2) return p.M > 1 && (p.M <= 4 || two) ? 26 : 0;
+    if (BITS == 4) return p.M == 4 || (p.M > 4 && two) ? 25 : 0;
+    return p.M > 4 && two && (p.M > 8 || w <= 256) ? 25 : 0;
+  }
+  // Two workgroups of wider codes do not fit a CU (INT4, K 5120, N 12288, M =
+  // 16: 12.4 against 11.5; more groups than 40 still gain, and so does a stream
+  // of more than three rounds above 8 rows, K 4096, N 14336 11.0 against 12.6),
+  // and INT8 gains only while every CU takes one (K 8192, N 12288: 25.0 against
+  // 21.8).
+  if (BITS == 2) return p.M > 8 && two ? 25 : 0;
+  if (BITS == 4) return p.M > 4 && two && (w <= 256 || (w > 384 && p.M > 8) || p.ng > 40) ? 25 : 0;
+  return p.M > 8 && two && w <= (p.ng > 40 ? 256 : 192) ? 25 : 0;
+}
+
 template <int BITS, int EPI>
 hipError_t launch_bits(const KParams& p, int variant, hipStream_t st) {
   constexpr int WNs = EPI == 0 ? 1 : 2;
@@ -1894,49 +1992,19 @@ hipError_t launch_bits(const KParams& p, int variant, hipStream_t st) {
     const int splitk_max = narrow ? (p.ng <= 16 ? 576 : 256) : 128;
     if (p.ng <= 24 && p.M <= splitk_max) variant = 0;
     else variant = narrow ? 4 : 5;
-    // The wide shapes (K >= 4096), M > 16 (K = 5120 and 17408, N = 5120, 7168
-    // and 2 x 17408, M = 17 .. 2160, us).  While the 64 x 64 blocks fit one
-    // round of the CUs they win by their shorter groups (K 5120 N 5120, M =
-    // 128: 15.2 against 21.6 of 32 x 128 and 32.1 of the tall 64 x 128), then
-    // 128 x 64 the same way (K 17408, M = 384: 85.5 against 97.2 of 64 x 64
-    // and 100.4 tall); beyond that the tall blocks, whose time per CU is
-    // about 31, 36 and 48 us for 1, 2 and 3 of 64 x 128 and 48 and 59 us for
-    // 1 and 2 of 64 x 256, in these rounds (M = 1024, N 5120: 48.2 and 59.5;
-    // N 7168: 73.7 and 59.3).  Up to 32 rows the 64-row blocks are half
-    // empty: the wide pair keeps 32 x 128 (M = 32: 30.1 against 37.2).
+    // the row blocks of the 27B-class shapes (K >= 4096; bench.py
+    // --gemm-variants-27b): 64 x 64 for the 136-group down projection, 128 x
+    // 64 from M = 1024, 32 x 256 for the others once M or N is large
+    if (p.K >= 4096 && p.M > 256) {
+      if (p.ng >= 96) variant = p.M >= 1024 ? 9 : 3;
+      else if (p.M >= 1024 || p.N >= 6144) variant = 6;
+    }
     if (p.K >= 4096 && p.M > 16) {
-      auto blocks = [&](long bm, long bn) { return ((p.M + bm - 1) / bm) * ((p.N + bn - 1) / bn); };
-      // Split K in turns while its blocks are few: 32 x 32 up to one workgroup
-      // per CU, at 2 bits two (INT4's registers allow one, so 64 x 32 there),
-      // and a little further where each row-block group is a longer chain
-      // (136 groups) or the 64-row blocks are half empty (M <= 32).  N 5120,
-      // K 5120: M = 32 13.9 -> 7.8 us, 96 14.3 -> 11.6, 128 14.7 against
-      // 16.3 (row blocks kept); K 17408: M = 32 47.4 -> 17.7, 96 49.1 -> 29.1,
-      // 128 50.4 -> 42.5, 192 54 against 58; the wide pair M = 32 30.6 ->
-      // 27.7; INT4 K 17408: M = 32 59.5 -> 20.5, 64 66.9 -> 34.3.
-      const long b32 = blocks(32, 32);
-      int tv = -1;
-      if (b32 <= 256 || (BITS == 2 && b32 <= (p.ng >= 96 ? 640 : 512)) || (p.M <= 32 && b32 <= 1152)) tv = 24;
-      else if (BITS != 2 && blocks(64, 32) <= 256) tv = 23;
-      if (tv >= 0) {
-        const hipError_t e = launch_bits<BITS, EPI>(p, tv, st);
-        if (e != hipErrorInvalidValue) return e;
-      }
-      int tall = -1;
-      if (blocks(64, 64) <= 256) variant = 3;
-      else if (blocks(128, 64) <= 256) variant = 9;
-      else if (p.M > 32) {
-        const long n21 = (blocks(64, 128) + 255) / 256, n22 = (blocks(64, 256) + 255) / 256;
-        const long t21 = 48 * (n21 / 3) + (n21 % 3 == 0 ? 0 : n21 % 3 == 1 ? 31 : 36);
-        const long t22 = 59 * (n22 / 2) + 48 * (n22 % 2);
-        tall = t22 < t21 ? 22 : 21;
-      }
-      if (tall >= 0) {  // a shape they cannot hold keeps the choice above
-        hipError_t e = launch_bits<BITS, EPI>(p, tall, st);
-        if (e == hipErrorInvalidValue && tall == 22) e = launch_bits<BITS, EPI>(p, 21, st);
-        if (e != hipErrorInvalidValue) return e;
-        if (p.M > 256) variant = p.ng >= 96 ? (p.M >= 1024 ? 9 : 3) : p.M >= 1024 || p.N >= 6144 ? 6 : variant;
-      }
+      int v = wide_shape<BITS>(p, variant);
+      hipError_t e = hipErrorInvalidValue;
+      if (v != variant) e = launch_bits<BITS, EPI>(p, v, st);
+      if (e == hipErrorInvalidValue && v == 22) e = launch_bits<BITS, EPI>(p, 21, st);
+      if (e != hipErrorInvalidValue) return e;  // else a shape it cannot hold keeps the choice above
     }
     // The mixed-iteration shapes (K of 8, 16 or 24 groups, 128 < M <= 1024;
     // bench.py --gemm-variants --gemm-mall, weights MALL-resident as in the
@@ -1960,28 +2028,19 @@ hipError_t launch_bits(const KParams& p, int variant, hipStream_t st) {
         if (e != hipErrorInvalidValue) return e;
       }
     }
-    // Decode rows on those shapes (bench.py --gemm-decode-27b, M = 1, 8, 16):
-    // the weight stream, for the plain projections two tiles per workgroup up
-    // to M = 4 and one above, one tile pair of 8 waves for the SwiGLU pair; its
-    // fold grows with the rows and its parked d with rows and depth, so split K
-    // in turns takes over above 8 rows (M = 16, us: QKV 7.3 -> 6.7, O 7.2 ->
-    // 6.6, gate/up 27.5 -> 21.8, INT4 38.0 -> 28.8), INT4 above 4 for the plain
-    // projections (M = 8: QKV 7.9 -> 7.6, O 7.8 -> 7.4; M = 4 7.15 against 7.6),
-    // and on the deep down projection above one row with 16 waves (M = 4 13.4 ->
-    // 11.7, 16 20.3 -> 12.5, M = 1 11.5 against 11.7; 8 waves 14.5), INT4 above 3
-    // with 8 waves, whose codes fit the registers (M = 4 16.7 -> 16.0, 16 waves
-    // 16.5; M = 8 20.4 -> 16.0; M = 2 15.4 against 16.0).  16-column blocks (320
-    // workgroups for down) lose: 14.0 with 8 waves, 17.4 with 16.  A shape a
-    // variant cannot hold (registers or LDS for wider codes) falls back to the
-    // next one, then to the choice above.
+    // Decode rows on the wide shapes: the weight stream (bench.py
+    // --gemm-decode-27b, M = 1, 8, 16), for the plain projections two 16-column
+    // tiles per workgroup up to M = 4 and one above, for the SwiGLU pair one
+    // tile pair of 8 waves up to M = 8 and then the row blocks; or split K in
+    // turns where decode_turns says so.  A shape a variant cannot hold
+    // (registers or LDS for wider codes) falls back to the next one, then to
+    // the choice above.
     if (p.K >= 4096 && p.M <= 16) {
       hipError_t e = hipErrorInvalidValue;
-      const bool deep = EPI == 0 && p.ng >= 96;
-      const int turns_above = deep ? (BITS == 2 ? 1 : BITS == 4 ? 3 : 4) : BITS == 4 && EPI == 0 ? 4 : 8;
-      if (p.M > turns_above) e = launch_bits<BITS, EPI>(p, deep && BITS != 4 ? 26 : 25, st);
+      if (const int v = decode_turns<BITS, EPI>(p)) e = launch_bits<BITS, EPI>(p, v, st);
       if (e != hipErrorInvalidValue) return e;
       if (EPI == 1) {
-        e = launch_bits<BITS, EPI>(p, 14, st);
+        if (p.M <= 8) e = launch_bits<BITS, EPI>(p, 14, st);
       } else {
         if (p.M <= 4) e = launch_bits<BITS, EPI>(p, 15, st);
         else if (p.ng < 96) e = launch_bits<BITS, EPI>(p, 14, st);

@@ -653,3 +653,51 @@ def test_qgemm_default_few_deep_rows(dev, bits):
             for b in (qd, sd, gd, od):
                 b.free()
         L.ifr_linear_free(dev.ctx, dl)
+
+
+# (bits, N, K, gate/up pair, general zeros, row counts): both sides of each line
+# of the default choice for K >= 4096
+WIDE_CASES = [(2, 5120, 4096, 0, 0, (9, 32, 33, 96, 97, 128, 512, 640)), (2, 4096, 4096, 0, 0, (9, 16, 160)),
+              (2, 4112, 5248, 0, 0, (8, 9, 17, 257)), (2, 12288, 4096, 0, 1, (160, 193, 385)),
+              (2, 7168, 5248, 0, 0, (160, 256)), (2, 3072, 12288, 0, 0, (4, 5, 192, 256)),
+              (2, 11008, 4096, 1, 0, (8, 9, 32, 33, 129)), (2, 16400, 4096, 1, 0, (17, 33)),
+              (4, 5120, 4096, 0, 0, (5, 32, 33, 64, 65, 160)), (4, 6144, 4096, 0, 1, (160, 320)),
+              (4, 5120, 8192, 0, 0, (4, 5, 65, 129)), (4, 8208, 4096, 0, 0, (4, 5, 16)),
+              (4, 4112, 12288, 0, 0, (3, 4, 5, 16)), (4, 12304, 4096, 1, 0, (9, 16, 32)),
+              (8, 5120, 5120, 0, 0, (8, 9, 32, 64, 128, 384)), (8, 6160, 4096, 0, 0, (9, 16, 160)),
+              (8, 4112, 12288, 0, 0, (4, 5, 8, 9)), (8, 8208, 4096, 1, 0, (9, 32, 33))]
+
+
+@pytest.mark.parametrize("case", range(len(WIDE_CASES)))
+def test_qgemm_default_wide_shapes(dev, case):
+    """The default choice on the wide shapes against the 32 x 128 row blocks,
+    bit for bit (every shape folds the groups in one order)."""
+    bits, N, K, pair, general, Ms = WIDE_CASES[case]
+    rng = np.random.default_rng(1000 + case)
+    zero = rng.uniform(0, (1 << bits) - 1, size=(N, K // 128)) if general else None
+    lins = [ia.make_linear(N, K, bits, rng, zero=zero) for _ in range(1 + pair)]
+    dl = C.c_void_p()
+    if pair:
+        ia.check(L.ifr_linear_upload_pair(dev.ctx, C.byref(lins[0].struct), C.byref(lins[1].struct), C.byref(dl)), "pair")
+    else:
+        ia.check(L.ifr_linear_upload(dev.ctx, C.byref(lins[0].struct), C.byref(dl)), "upload")
+    try:
+        for M in Ms:
+            q = rng.integers(-127, 128, size=(M, K), dtype=np.int8)
+            g = q.reshape(M, K // 128, 128).sum(2, dtype=np.int32).astype(np.float32)
+            qd, sd, gd = dev.upload(ia.atile(q)), dev.upload(rng.uniform(1e-3, 1e-2, M).astype(np.float32)), dev.upload(g)
+            od = dev.alloc(M * N * 2)
+            announce(f"wide default bits={bits} N={N} K={K} pair={pair} M={M}")
+            args = (qd.p, sd.p, gd.p, M, od.p)
+            ia.check(L.ifr_quant_gemm_variant(dev.ctx, dl, *args, 5), "32 x 128")
+            ref = dev.download(od, np.uint16, (M, N))
+            ia.check(L.ifr_memset(dev.ctx, od.p, 0xFF, M * N * 2), "memset")
+            if pair:
+                ia.check(L.ifr_quant_gemm_swiglu(dev.ctx, dl, *args), "default")
+            else:
+                ia.check(L.ifr_quant_gemm(dev.ctx, dl, *args, None), "default")
+            assert np.array_equal(dev.download(od, np.uint16, (M, N)), ref), M
+            for b in (qd, sd, gd, od):
+                b.free()
+    finally:
+        L.ifr_linear_free(dev.ctx, dl)
