@@ -337,9 +337,11 @@ __global__ __launch_bounds__(512) void row_quant1024_kernel(RowQuantArgs a) {
 // so the result is bit-identical to the LDS kernel it replaces.
 // Bound by its chain of exchanges and the RMS chains (K / 8 dependent fused
 // steps), not by memory, so a wide row (K >= 4096) takes 1024 threads while
-// the rows leave CUs idle, and the chains read ahead: K 5120, normed and
-// rotated, one row 10.6 -> 9.1 us, 2160 rows 36.8 -> 35.7 (of which 17.3 without
-// norm and rotation).
+// the rows leave CUs idle: K 5120, normed and rotated, one row 10.6 -> 9.1
+// us, 2160 rows (256 threads) 35.1 -> 33.1, of which 17.0 without norm and rotation.
+// (The chains' reads are left to the compiler, which keeps 16 of them in flight;
+// a loop that names the next reads ahead of the sums compiles to 8 and a wait
+// for them: 0.3 to 0.6 us longer.)
 template <int M, int E>
 __device__ __forceinline__ void bfly_lanes(float (&v)[E]) {
 #pragma unroll
@@ -525,14 +527,10 @@ __global__ __launch_bounds__(T) void row_quant_wide(RowQuantArgs a) {
     if (t < 8) {
       float acc = 0.0f;
       const float4* xc = reinterpret_cast<const float4*>(xs + t * CS);
-      // the next eight float4 are read while these eight are summed
-      float4 x8[8], y8[8];
-#pragma unroll
-      for (int i = 0; i < 8; ++i) x8[i] = xc[i];
       for (int n4 = 0; n4 < K / 32; n4 += 8) {
-        const int nn = min(n4 + 8, K / 32 - 8);
+        float4 x8[8];
 #pragma unroll
-        for (int i = 0; i < 8; ++i) y8[i] = xc[nn + i];
+        for (int i = 0; i < 8; ++i) x8[i] = xc[n4 + i];
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
           acc = fmaf(x8[i].x, x8[i].x, acc);
@@ -540,8 +538,6 @@ __global__ __launch_bounds__(T) void row_quant_wide(RowQuantArgs a) {
           acc = fmaf(x8[i].z, x8[i].z, acc);
           acc = fmaf(x8[i].w, x8[i].w, acc);
         }
-#pragma unroll
-        for (int i = 0; i < 8; ++i) x8[i] = y8[i];
       }
       red[t] = acc;
     }
@@ -1243,9 +1239,12 @@ hipError_t launch_row_quant(const RowQuantArgs& a, hipStream_t st) {
     while (2 * P <= a.K) P *= 2;
     const int et = (a.K - P) / 256;
     if (a.K % 256 == 0 && (et & (et - 1)) == 0) {
-      // 1024 threads a row while every row has a CU to itself (K 5120, M = 256:
-      // 11.8 -> 11.0 us; two rows a CU lose: M = 537 16.1 against 21.0)
-      const bool wide = a.M <= 256 && et % 4 == 0;
+      // 1024 threads a row while every row has a CU to itself (K 5120, normed and
+      // rotated, M = 256: 12.2 -> 10.7 us; two rows a CU lose: M = 537 16.1 against
+      // 21.0), except 64-wide scales over a tail without a rotation, which has
+      // only their lane groups to widen (K 5120 7.1 against 7.3, 6144 7.5 against 8.0)
+      const bool fwht = a.rotate || (a.src == SRC_RESID && a.rot_y);
+      const bool wide = a.M <= 256 && et % 4 == 0 && (fwht || a.ga == 0 || et == 0);
       const dim3 grid(a.M);
       switch (P / 256) {
         case 1: hipLaunchKernelGGL((row_quant_wide<1, 256>), grid, dim3(256), 0, st, a); return hipGetLastError();

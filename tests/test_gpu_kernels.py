@@ -585,7 +585,8 @@ def test_qgemm_turns_edges(dev, bits, zmode):
 
 
 @pytest.mark.parametrize("K,norm,rot,rnd,ga", [(4096, 1, 1, 0, 0), (5120, 1, 1, 0, 0), (5120, 1, 1, 1, 64),
-                                               (6144, 1, 1, 0, 0), (8192, 1, 1, 0, 64), (4352, 1, 1, 0, 0)])
+                                               (6144, 1, 1, 0, 0), (8192, 1, 1, 0, 64), (4352, 1, 1, 0, 0),
+                                               (5120, 1, 0, 1, 64), (6144, 1, 0, 0, 64), (8192, 1, 0, 1, 64)])
 def test_act_quant_wide_rows_few_and_many(dev, K, norm, rot, rnd, ga):
     """Rows of 4096 columns and more on both sides of the 256 rows up to which
     a row takes 1024 threads (K = 4352: never, its tail does not divide), bit
