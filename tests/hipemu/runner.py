@@ -488,31 +488,36 @@ def forward_fused_qk():
 
 @scenario
 def gemm_f16():
-    """The FP16-activation dequant GEMM (both kernels: M == 1 and tiled) in
-    bounds and bit-exact against the oracle, INT2 / INT4 / INT8."""
+    """The FP16-activation dequant GEMM in bounds and bit-exact against the
+    oracle, INT2 / INT4 / INT8: one row, each row-block size the launch picks
+    (16, 32 and 64 rows, the last with more than 64 KB of LDS), partial last
+    blocks and column tiles, activations off a 16-byte boundary."""
     import intfer_amd as ia
     from oracle import pyoracle as po
     L = ia.lib()
     dev = ia.Device(0)
     rng = np.random.default_rng(17)
     for bits in (2, 4, 8):
-        N, K = 80, 256
-        lin = ia.make_linear(N, K, bits, rng)
-        dl = C.c_void_p()
-        ia.check(L.ifr_linear_upload(dev.ctx, C.byref(lin.struct), C.byref(dl)), "upload")
-        for M in (1, 3, 70):
-            a = (rng.standard_normal((M, K)) * 2).astype(np.float16)
-            ad, od = dev.upload(a.view(np.uint16)), dev.alloc(M * N * 2)
-            ia.check(L.ifr_quant_gemm_f16(dev.ctx, dl, ad.p, M, C.c_float(0.5), od.p), "f16")
-            got = dev.download(od, np.uint16, (M, N))
-            ref = np.empty((M, N), np.uint16)
-            po.oracle().or_qgemm_f16(po.ptr(a.view(np.uint16)), M, C.byref(lin.struct), np.float32(0.5),
-                                     po.ptr(ref))
-            assert np.array_equal(got, ref), (bits, M)
-            ad.free()
-            od.free()
-        L.ifr_linear_free(dev.ctx, dl)
-        say(f"fp16 GEMM bits={bits}: M = 1, 3, 70 bit-exact")
+        # 1040 columns are 17 column blocks: 32-row blocks take fewer rounds of the
+        # 256 CUs at 250 rows, 64-row blocks at 784
+        for N, K, Ms in ((80, 256, ((1, 0), (3, 0), (70, 2))), (1040, 128, ((250, 0), (784, 2)))):
+            lin = ia.make_linear(N, K, bits, rng)
+            dl = C.c_void_p()
+            ia.check(L.ifr_linear_upload(dev.ctx, C.byref(lin.struct), C.byref(dl)), "upload")
+            for M, off in Ms:
+                a = (rng.standard_normal((M, K)) * 2).astype(np.float16)
+                ad = dev.upload(np.concatenate([np.zeros(off // 2, np.uint16), a.view(np.uint16).reshape(-1)]))
+                od = dev.alloc(M * N * 2)
+                ia.check(L.ifr_quant_gemm_f16(dev.ctx, dl, C.c_void_p(ad.p.value + off), M, C.c_float(0.5), od.p), "f16")
+                got = dev.download(od, np.uint16, (M, N))
+                ref = np.empty((M, N), np.uint16)
+                po.oracle().or_qgemm_f16(po.ptr(a.view(np.uint16)), M, C.byref(lin.struct), np.float32(0.5),
+                                         po.ptr(ref))
+                assert np.array_equal(got, ref), (bits, N, M)
+                ad.free()
+                od.free()
+            L.ifr_linear_free(dev.ctx, dl)
+            say(f"fp16 GEMM bits={bits} N={N} K={K}: rows {[m for m, _ in Ms]} bit-exact")
     dev.close()
 
 
@@ -720,14 +725,16 @@ def act_quant():
     dev = ia.Device(0)
     # 1024 has its own kernel; the register kernel takes every K whose tail
     # per thread is 0 or a power of two (P = floor_pow2(K)): 256, 512, 768,
-    # 1280, 2048, 2304, 3072, 5120, 6144, 8192; 1792 (tail 3) takes the LDS one
-    for (K, norm, rot, rnd, ga) in [(1024, 1, 1, 0, 0), (1024, 0, 0, 1, 64), (2048, 0, 0, 0, 0),
+    # 1280, 2048, 2304, 3072, 5120, 6144, 8192; 1792 (tail 3) takes the LDS one.
+    # From 4096 on a row takes 1024 threads up to 256 rows (257 here: 256
+    # threads), and 64-wide scales over an unrotated tail always 256
+    for (K, norm, rot, rnd, ga, M) in [(*c, 19) for c in [(1024, 1, 1, 0, 0), (1024, 0, 0, 1, 64), (2048, 0, 0, 0, 0),
                                     (3072, 1, 0, 0, 0), (5120, 1, 1, 0, 0), (256, 1, 1, 0, 0),
                                     (512, 1, 1, 0, 64), (768, 1, 1, 0, 0), (1280, 1, 1, 1, 64),
                                     (2304, 1, 1, 0, 0), (5120, 1, 1, 1, 64), (6144, 1, 1, 0, 0),
-                                    (8192, 0, 1, 0, 64), (1792, 1, 1, 0, 0)]:
+                                    (8192, 0, 1, 0, 64), (1792, 1, 1, 0, 0), (5120, 1, 0, 1, 64)]] + [
+                                       (5120, 1, 1, 0, 0, 257), (8192, 1, 1, 0, 64, 257)]:
         rng = np.random.default_rng(K)
-        M = 19
         x = (rng.standard_normal((M, K), dtype=np.float32) * 2.5).astype(np.float32)
         w = rng.normal(0, 0.1, size=K).astype(np.float32)
         q, s, g = po.act_quant(x, norm_w=w if norm else None, rotate=rot, round=rnd, ga=ga)
@@ -741,7 +748,7 @@ def act_quant():
         assert np.array_equal(qg, q), K
         assert np.array_equal(dev.download(sd, np.float32, (M, ns)).view(np.uint32), s.view(np.uint32)), K
         assert np.array_equal(dev.download(gd, np.float32, (M, K // 128)), g), K
-        say(f"act_quant K={K} norm={norm} rot={rot} round={rnd} ga={ga} ok")
+        say(f"act_quant K={K} norm={norm} rot={rot} round={rnd} ga={ga} M={M} ok")
     dev.close()
 
 

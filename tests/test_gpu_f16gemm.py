@@ -84,3 +84,43 @@ def test_qgemm_f16_row_blocks_and_unaligned_rows(dev, bits, N, K, M, shift):
         ad.free()
         od.free()
         L.ifr_linear_free(dev.ctx, dl)
+
+
+@pytest.mark.parametrize("bits", [2, 4, 8])
+@pytest.mark.parametrize("M", [1, 2, 100])
+def test_qgemm_f16_rounding_of_every_step(dev, bits, M):
+    """The second half of a row meets the first half's weights negated, so the
+    exact sums are 0 and an output is what the roundings of its 512 steps left:
+    it pins the order of the products inside and between the matrix
+    instructions and the single rounding of each step (fp32 weights at one
+    row).  fp16 subnormal activations among them."""
+    rng = np.random.default_rng(70 + bits)
+    N, K = 48, 512
+    half = ia.make_linear(N, K // 2, bits, rng, scale_sigma=0.5)
+    vals = np.concatenate([half.values, ((1 << bits) - 1) - half.values], 1)
+    twice = lambda x: np.concatenate([x.reshape(N, -1)] * 2, 1)
+    lin = ia.HostLinear(N, K, bits, ia.pack_codes(vals, bits), twice(half.scale), twice(half.zero), vals, 0.0)
+    a = rng.standard_normal((M, K // 2)) * 10.0 ** rng.integers(-3, 4, size=(M, K // 2))
+    a[:, ::16] *= 1e-6
+    a = np.concatenate([a, a], 1).astype(np.float16)
+    assert ((a != 0) & (np.abs(a) < 6.1e-5)).any()
+    alpha = np.float32(3.7)
+    ref, rev = np.empty((M, N), np.uint16), np.empty((M, N), np.uint16)
+    po.oracle().or_qgemm_f16(ptr(a.view(np.uint16)), M, C.byref(lin.struct), alpha, ptr(ref))
+    # the test can tell orders apart: the halves swapped sum to something else
+    b = np.ascontiguousarray(a[:, ::-1])
+    back = ia.HostLinear(N, K, bits, ia.pack_codes(np.ascontiguousarray(vals[:, ::-1]), bits), twice(half.scale)[:, ::-1].copy(),
+                         lin.zero, vals, 0.0)
+    po.oracle().or_qgemm_f16(ptr(b.view(np.uint16)), M, C.byref(back.struct), alpha, ptr(rev))
+    assert (ref != rev).mean() > 0.5
+    dl = C.c_void_p()
+    ia.check(L.ifr_linear_upload(dev.ctx, C.byref(lin.struct), C.byref(dl)), "upload")
+    ad, od = dev.upload(a.view(np.uint16)), dev.alloc(M * N * 2)
+    try:
+        announce(f"fp16 GEMM rounding bits={bits} M={M}")
+        ia.check(L.ifr_quant_gemm_f16(dev.ctx, dl, ad.p, M, C.c_float(alpha), od.p), "f16 gemm")
+        assert np.array_equal(dev.download(od, np.uint16, (M, N)), ref)
+    finally:
+        ad.free()
+        od.free()
+        L.ifr_linear_free(dev.ctx, dl)

@@ -44,3 +44,31 @@ def test_fused_qk_epilogue_bit_identical(dev, kv8, qkn):
             assert np.array_equal(a, b)
     finally:
         m.close()
+
+
+def test_fused_qk_epilogue_wide_rows(dev):
+    """hidden 5120, 40 heads: the epilogue's 32 x 128 row blocks against the two
+    passes, whose plain projection takes another launch shape at every one of
+    these row counts (split K in turns, 64 x 64 blocks, the weight stream)."""
+    cfg = ia.default_cfg(hidden=5120, layers=1, n_heads=40, n_kv=8, inter=256, vocab=512)
+    m = ia.SynthModel(cfg, seed=18, bits=2)
+    try:
+        outs = []
+        for sep in (0, 1):
+            eng = ia.Engine(dev, m, max_seqs=2, max_seq_tokens=512, pool_tokens=2 * 512, max_rows=300, separate_qk=sep)
+            rng = np.random.default_rng(32)
+            got = []
+            for M in (16, 17, 32, 112, 256, 257):
+                announce(f"fused q/k epilogue, hidden 5120, {M} rows, separate={sep}")
+                s = eng.seq_open()
+                eng.set_timing(True)
+                toks = rng.integers(0, cfg.vocab, size=M)
+                got.append(eng.forward([(s, p, int(t), ia.ROW_PREFILL, 1) for p, t in enumerate(toks)], logits=True)[1])
+                assert (eng.timing("qk_rope_kv")[1] == 0) == (sep == 0 and 16 < M <= 256), M
+                eng.set_timing(False)
+                eng.seq_close(s)
+            outs.append(got)
+        for a, b in zip(*outs):
+            assert np.array_equal(a, b)
+    finally:
+        m.close()
