@@ -1859,29 +1859,6 @@ hipError_t launch_rows_r(const KParams& p, hipStream_t st) {
 template <int BITS, int EPI>
 hipError_t launch_bits(const KParams& p, int variant, hipStream_t st);
 
-// The QKV projection with the q/k epilogue: the default shape when it is a
-// 32 x 128 row block (one head per workgroup), else declined (the caller
-// runs the GEMM and the separate q/k pass).
-template <int BITS>
-hipError_t launch_bits_qk(const KParams& p, int variant, hipStream_t st) {
-  if (variant < 0) {
-    const int ng = p.ng;
-    // the plain-GEMM heuristic of launch_bits for these shapes
-    variant = (ng <= 24 && p.M <= 128) ? 0 : 5;
-    if (p.K >= 4096 && p.M > 256 && (ng >= 96 || p.M >= 1024 || p.N >= 6144)) variant = -1;
-    if (p.K >= 4096 && p.M <= 16) variant = -1;
-    // (the whole-K 32 x 128 block, variant 17, holds the epilogue at 234
-    // VGPRs against 126 here: slower in the serve load, 12.7 -> 13.4 us)
-  }
-  switch (variant) {
-    case 4: return launch_rows_r<BITS, 2, 2, 1, 4, 2>(p, st);
-    case 5: return launch_rows_r<BITS, 2, 2, 1, 2, 2>(p, st);
-    case 12: return launch_rows_r<BITS, 2, 2, 1, 8, 2>(p, st);
-    case 17: return launch_full<BITS, 2, 2, 1, 2>(p, st);
-    default: return hipErrorInvalidValue;
-  }
-}
-
 // The wide shapes (K >= 4096), M > 16: split K in turns (23, 24), 64 x 64 or
 // 128 x 64 blocks (3, 9), the tall blocks (21, 22) or `rows`, the row blocks of
 // launch_bits.  The lines were placed over K 4096 .. 17408, N 1024 .. 28672,
@@ -1940,6 +1917,40 @@ int wide_shape(const KParams& p, int rows) {
   const long t21 = 48 * (n21 / 3) + (n21 % 3 == 0 ? 0 : n21 % 3 == 1 ? 31 : 36);
   const long t22 = 59 * (n22 / 2) + 48 * (n22 % 2);
   return t22 < t21 ? 22 : 21;
+}
+
+// The QKV projection with the q/k epilogue in its 32 x 128 row blocks (one head
+// per workgroup), else declined (the caller runs the plain projection and the
+// q/k pass): for few rows on a short K, whose split-K shape has no epilogue, by
+// the plain GEMM's choice there; on the wide shapes (K >= 4096) for the weight
+// stream's rows, for many, and where the plain projection splits K in turns or,
+// at 2 bits, takes 64 x 64 blocks, which save more than the pass costs (a whole
+// layer with a small MLP, hidden 5120, 40 heads, us, the two passes against
+// the epilogue: M = 32 81.6 / 98.0, 64 92.5 / 105.1, 128 109.1 / 116.6; with row
+// blocks in both, M = 192, 128.6 / 124.4; INT4 M = 64 97.2 / 107.1, 112 116.5 /
+// 117.8; INT8 M = 64 104.4 / 114.3, 112 131.2 / 127.8).
+template <int BITS>
+hipError_t launch_bits_qk(const KParams& p, int variant, hipStream_t st) {
+  if (variant < 0) {
+    const int ng = p.ng;
+    variant = (ng <= 24 && p.M <= 128) ? 0 : 5;
+    if (p.K >= 4096) {
+      if (p.M <= 16 || (p.M > 256 && (ng >= 96 || p.M >= 1024 || p.N >= 6144))) variant = -1;
+      else if (p.M <= 256) {
+        const int plain = wide_shape<BITS>(p, 5);
+        if (plain == 23 || plain == 24 || (BITS == 2 && plain == 3)) variant = -1;
+      }
+    }
+    // (the whole-K 32 x 128 block, variant 17, holds the epilogue at 234
+    // VGPRs against 126 here: slower in the serve load, 12.7 -> 13.4 us)
+  }
+  switch (variant) {
+    case 4: return launch_rows_r<BITS, 2, 2, 1, 4, 2>(p, st);
+    case 5: return launch_rows_r<BITS, 2, 2, 1, 2, 2>(p, st);
+    case 12: return launch_rows_r<BITS, 2, 2, 1, 8, 2>(p, st);
+    case 17: return launch_full<BITS, 2, 2, 1, 2>(p, st);
+    default: return hipErrorInvalidValue;
+  }
 }
 
 // Split K in turns for M <= 16 on the wide shapes (8 waves: 25, 16 waves: 26),
