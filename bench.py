@@ -501,8 +501,8 @@ def gemm_variants(ia, dev, Ms=(128, 256, 576, 1024), bits=2, reps=3, shapes=SHAP
     MALL); one line per (shape, M, variant).  With rotate_bytes = 100e6 the
     copies stay in the MALL but not in L2, as the 0.8B model's weights do in
     the serve load (28 layers x 4.4 MB, each touched once per iteration).
-    rows: A also passed row-major (ifr_quant_gemm_rows; the weight stream
-    stages its A rows from it at M <= 4)."""
+    rows: A also passed row-major (ifr_quant_gemm_rows; the weight stream,
+    variants 13 to 15, stages its A rows from it at M <= 4)."""
     import ctypes as C
     L = ia.lib()
     rng = np.random.default_rng(0)

@@ -241,10 +241,11 @@ int ifr_quant_gemm_variant(ifr_ctx* ctx, const ifr_dlinear* w, const int8_t* a_d
 /* No counterpart in the reference (its activation codes have one layout):
  * ifr_quant_gemm (plain linear) or ifr_quant_gemm_swiglu (gate/up pair) with
  * the activation codes also given row-major, arow_d int8 [M][K] (the codes of
- * a_d's M rows, unpadded).  The decode weight stream (M <= 4, K >= 4096)
- * stages its A rows from arow_d, K contiguous bytes per row, where in the
- * A-tile layout a row holds 16 of every 128 bytes it touches; every other
- * launch shape reads a_d.  arow_d may be NULL.  variant: -1 for the size
+ * a_d's M rows, unpadded).  The decode weight stream stages its A rows from
+ * arow_d at M <= 4, K >= 4096, K contiguous bytes per row, where in the A-tile
+ * layout a row holds 16 of every 128 bytes it touches; every other launch shape
+ * reads a_d, also the one that the heuristic takes instead of the stream for K
+ * >= 12288 above one row at 2 bits and above three at 4.  arow_d may be NULL.  variant: -1 for the size
  * heuristic, else a launch shape as in ifr_quant_gemm_variant (IFR_EDECLINE
  * where it does not apply).  The bits are those of ifr_quant_gemm. */
 int ifr_quant_gemm_rows(ifr_ctx* ctx, const ifr_dlinear* w, const int8_t* a_d,
@@ -262,7 +263,7 @@ int ifr_quant_gemm_rows(ifr_ctx* ctx, const ifr_dlinear* w, const int8_t* a_d,
  * [M][K] row-major, out_d fp16 [M][N]; alpha is the tensor's global factor
  * (1 when it has none).  IFR_EDECLINE for a gate/up pair, a linear whose
  * zeros are not all C/2 (the reference path knows only the codebook), or
- * K > 32768 at M == 1. */
+ * K > 32768 at M == 1 (a bound of this interface, not of the kernel). */
 int ifr_quant_gemm_f16(ifr_ctx* ctx, const ifr_dlinear* w, const uint16_t* a_d, int32_t M,
                        float alpha, uint16_t* out_d);
 

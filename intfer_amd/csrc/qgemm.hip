@@ -876,10 +876,11 @@ __global__ __launch_bounds__(256) void qgemm_full(KParams p) {
 // memory unit moves each A byte once per workgroup; a wave's codes and scale |
 // zero pairs of two groups are in flight in registers, each slot refilled as
 // soon as its column tile is unpacked, with plain loads (the other row blocks
-// read them from the L2: streaming loads 577, plain 530 us).  Same fold, same
-// group order, same bits.  Against qgemm_rows at M = 2160 (INT2): gate/up
-// 5120 -> 2 x 17408 642 -> 530 us, down 17408 -> 5120 455 -> 300, QKV 146 -> 116,
-// O 108 -> 95; INT4 at M = 1024: gate/up 436 -> 307, down 275 -> 170.
+// read them from the L2: streaming loads lose 9 %).  Same fold, same group
+// order, same bits.  Against qgemm_rows (the launch alone, back to back on
+// weights from HBM, HIP events) at M = 2160 (INT2): gate/up 5120 -> 2 x 17408
+// 626 -> 497 us (1.55 POP/s), down 17408 -> 5120 459 -> 274, QKV 147 -> 108, O 109
+// -> 88; INT4 at M = 1024: gate/up 418 -> 289, down 274 -> 155.
 template <int BITS, int WM, int WN, int EPI, bool FF>
 __global__ __launch_bounds__(256, 2) void qgemm_tall(KParams p) {
   constexpr int BM = 16 * WM, BN = 64 * WN, SP = BM + 4;
@@ -1332,8 +1333,8 @@ __global__ __launch_bounds__(64 * NWV) void qgemm_stream(KParams p) {
 // of two are in flight in registers; S (FF: the MFMA's start value, whose bits
 // make the result read as 1.5 * 2^23 + 2T - C S) and the scale | zero pairs
 // of a turn are staged in LDS, four buffers.
-// Down 17408 -> 5120, INT2, 32 rows 47.4 -> 17.7 us, 16 rows (16 waves) 20.3 ->
-// 12.7; O 5120 -> 5120, 32 rows 13.9 -> 7.8.
+// Down 17408 -> 5120, INT2, weights from HBM: 32 rows 67.1 -> 18.1 us, 16 rows
+// (16 waves) 20.0 -> 12.7; O 5120 -> 5120, 32 rows 22.1 -> 8.1.
 template <int BITS, int WM, int WN, int NWV, int EPI, bool FF>
 __global__ __launch_bounds__(64 * NWV) void qgemm_turns(KParams p) {
   constexpr int BM = 16 * WM, BN = 16 * WN, TT = WM * WN, NT = 64 * NWV, SP = BM + 4;

@@ -952,8 +952,9 @@ __device__ __forceinline__ int pack_group_of(const uint16_t* nblk, int ngroups, 
 // once, into registers (k < R = kPackRowsPerThread); every later phase
 // works from those registers and six LDS arrays, and every loop runs over
 // rows, groups or q-blocks in parallel (no thread walks a group's q-blocks
-// or quads).  Ten barriers in all.  LDS arrays, one map per phase (the
-// three index maps, all <= 6144, in 16 bits: 159.9 KB at M = 6144):
+// or quads).  Ten barriers in all, twelve with the records staged.  LDS
+// arrays, one map per phase (the three index maps, all <= 6144, in 16 bits:
+// 159.9 KB at M = 6144):
 //   fs, fw  group-start / want flags of row m (scanned: starts / wants before
 //           m), then the per-q-block dispatch-slot counts (scanned)
 //   gpos    first KV position of group g
@@ -963,7 +964,7 @@ __device__ __forceinline__ int pack_group_of(const uint16_t* nblk, int ngroups, 
 //   nblk    first q-block of group g (nb at ngroups)    16 bits
 //   bgrp    group of q-block b                          16 bits
 constexpr int kPackThreads = 1024, kPackRowsPerThread = 6, kPackMaxRows = kPackThreads * kPackRowsPerThread;
-// The ten barriers and the chain of loads and stores between them are what a
+// The barriers and the chain of loads and stores between them are what a
 // small batch waits for (6.8 us at one row, 7.7 at 512), not its work, so up to
 // 512 rows 4 workgroups of 4 waves take it and read each record once, in order,
 // through LDS: the records can then stay in host memory, without the copy
