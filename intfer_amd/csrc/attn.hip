@@ -355,10 +355,12 @@ __global__ __launch_bounds__(256) void attn_kernel(AttnArgs p, KVLayout kv) {
 // quantization (half-away) of the [nq*hd] attention row for the O projection.
 // Thread t owns the 8 consecutive dims [8 t, 8 t + 8) of the row (a chunk never
 // straddles a head; threads past nq*hd/8 idle), 256 threads up to 2048 columns,
-// 640 up to 5120, else 1024.  Bound by the latency of its dependent loads, so
-// a wide row gets more threads and not more columns a thread (40 heads, 60
-// rows: 32 columns a thread in 256 threads, two rounds of loads at 208 VGPRs,
-// 20.1 us; 640 threads 9.8 us).
+// 512 up to 4096, 640 up to 5120, else 1024.  Bound by the latency of its
+// dependent loads, so a wide row gets more threads and not more columns a thread
+// (64 rows of 1000 tokens, us: 40 heads 9.5 against 11.4 of 32 columns a thread
+// in 256 threads, of 2000 tokens 10.2 / 15.7), but no idle waves (32 heads: 512
+// threads 7.6, 640 threads 9.0, 16 columns in 256 threads 8.7; 512 rows in two
+// chunks 15.1 / 19.6 / 22.5).
 // The merge runs the splits in order: the max over all splits first, then l
 // and O accumulated split by split, loaded in rounds of 4 with clamped
 // (unconditional) indices so each round is one memory latency.
@@ -522,6 +524,7 @@ hipError_t launch_combine(const CombineArgs& a, hipStream_t st) {
   if (N % 128 != 0 || N > 256 * 32 || a.hd != kHD || !a.q || !a.qscale || !a.gsum)
     return hipErrorInvalidValue;
   if (N <= 256 * 8) hipLaunchKernelGGL(combine_kernel<256>, dim3(a.M), dim3(256), 0, st, a);
+  else if (N <= 512 * 8) hipLaunchKernelGGL(combine_kernel<512>, dim3(a.M), dim3(512), 0, st, a);
   else if (N <= 640 * 8) hipLaunchKernelGGL(combine_kernel<640>, dim3(a.M), dim3(640), 0, st, a);
   else hipLaunchKernelGGL(combine_kernel<1024>, dim3(a.M), dim3(1024), 0, st, a);
   return hipGetLastError();

@@ -506,9 +506,9 @@ def test_qgemm_tall_blocks_odd_depths(dev, bits, zmode):
     run(16448, 4224, (33, 200), vs_blocks)
 
 
-@pytest.mark.parametrize("heads", [24, 48, 64])
+@pytest.mark.parametrize("heads", [24, 32, 40, 48, 64])
 def test_attention_row_widths(dev, heads):
-    """Rows of 3072, 6144 and 8192 attention columns (the combine's 640- and
+    """Rows of 3072 to 8192 attention columns (the combine's 512-, 640- and
     1024-thread rows, partly idle and full), short and beyond the 8 KV splits
     merged in one round."""
     cfg = ia.default_cfg(layers=1, vocab=512, hidden=256, inter=256, n_heads=heads)
