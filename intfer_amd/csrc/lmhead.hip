@@ -32,7 +32,7 @@ __device__ __forceinline__ bool better(float v, int i, float bv, int bi) {
   return v > bv || (v == bv && i < bi);
 }
 
-template <int WM>
+template <int WM, int R>
 __global__ __launch_bounds__(256) void lmhead_kernel(LmP p) {
   extern __shared__ float as_l[];  // [16 WM rows][nsteps] activation scales of the block
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -64,8 +64,7 @@ __global__ __launch_bounds__(256) void lmhead_kernel(LmP p) {
   // (L2).  One step at a time reaches the stream's rate while many waves share a
   // SIMD (32 rows with the argmax reduce: 38.7 us, with 4 steps 47.8); the
   // 64-row block holds fewer and needs them: 64 rows 76.3 -> 64.6 us, of which
-  // the reduce is 5.
-  constexpr int R = WM == 4 ? 4 : 1;
+  // the reduce is 5 (launch_lmhead: where its waves take no more rounds for it).
   v4i Bq[R][kWN];
   auto load_b = [&](v4i (&B)[kWN], int s) {
     s = min(s, p.nsteps - 1);
@@ -198,11 +197,11 @@ __global__ __launch_bounds__(1024) void argmax_final_kernel(const float* pv, con
   if (threadIdx.x == 0) best[row] = (bv > -1e30f) ? bi : -1;
 }
 
-template <int WM>
+template <int WM, int R>
 hipError_t launch_wm(const LmP& p, int nparts, int nrb, hipStream_t st) {
   const size_t lds = (size_t)16 * WM * p.nsteps * sizeof(float);
   if (lds > 64 * 1024) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(lmhead_kernel<WM>, dim3(nparts / 4, nrb), dim3(256), lds, st, p);
+  hipLaunchKernelGGL((lmhead_kernel<WM, R>), dim3(nparts / 4, nrb), dim3(256), lds, st, p);
   return hipGetLastError();
 }
 
@@ -222,10 +221,18 @@ hipError_t launch_lmhead(LmHeadArgs& a, hipStream_t st) {
   a.nparts = lmhead_nparts(a.V);
   LmP p{a.a, a.as, a.wcodes, a.wscale, a.logits, a.part_val, a.part_idx, a.W, a.V, a.H, a.H / 64};
   hipError_t e;
-  if (a.W <= 16) e = launch_wm<1>(p, a.nparts, 1, st);
-  else if (a.W <= 32) e = launch_wm<2>(p, a.nparts, 1, st);
-  else if (a.W <= 64) e = launch_wm<4>(p, a.nparts, 1, st);
-  else e = launch_wm<4>(p, a.nparts, (a.W + 63) / 64, st);
+  // Four steps in flight take 157 VGPRs: three waves a SIMD, 3072 on the chip,
+  // where one step holds four.  A round of three costs about 0.7 of one of
+  // four (0.8 at 16 K steps and fewer), so the whole rounds decide (us with the
+  // reduce, four steps / one: H 1024, V 32000, 192 rows' 3000 waves 37.8 / 40.9,
+  // 256 rows' 4000 waves 60.5 / 48.0; V 151936, 64 rows 64.4 / 76.5, 256 rows 197 /
+  // 188, and at H 2048 312 / 316).
+  const int nrb = (a.W + 63) / 64;
+  const long waves = (long)a.nparts * nrb, r3 = (waves + 3071) / 3072, r4 = (waves + 4095) / 4096;
+  if (a.W <= 16) e = launch_wm<1, 1>(p, a.nparts, 1, st);
+  else if (a.W <= 32) e = launch_wm<2, 1>(p, a.nparts, 1, st);
+  else if (r3 * (p.nsteps > 16 ? 7 : 8) <= r4 * 10) e = launch_wm<4, 4>(p, a.nparts, nrb, st);
+  else e = launch_wm<4, 1>(p, a.nparts, nrb, st);
   if (e != hipSuccess) return e;
   hipLaunchKernelGGL(argmax_final_kernel, dim3(a.W), dim3(1024), 0, st, a.part_val, a.part_idx,
                      a.nparts, a.W, a.best);

@@ -610,10 +610,11 @@ def test_act_quant_wide_rows_few_and_many(dev, K, norm, rot, rnd, ga):
     wd.free()
 
 
-@pytest.mark.parametrize("hidden,vocab", [(256, 528), (768, 140016)])
+@pytest.mark.parametrize("hidden,vocab", [(256, 528), (768, 140016), (768, 50272)])
 def test_lm_head_row_blocks(dev, hidden, vocab):
     """The lm_head where its row blocks end (64 rows: several K steps of
-    weights in flight, 4 steps and 12 here), on more and fewer partials a row
+    weights in flight, 4 steps and 12 here; one at 50272 columns and 65 rows,
+    whose waves four steps would put into a second round), on more and fewer partials a row
     than the argmax reduce reads in one pass.  Sequences of one token, whose
     attention is exact: tokens and logit rows bit for bit, up to a rare ulp of
     SwiGLU's device expf (test_single_token_sequences_bit_exact)."""
