@@ -18,6 +18,8 @@
 #include "ifr_dev.h"
 #include "ifr_kernels.h"
 
+#include <type_traits>
+
 namespace ifrk {
 namespace {
 
@@ -393,15 +395,17 @@ __global__ __launch_bounds__(NT) void combine_kernel(CombineArgs a) {
 #pragma unroll
   for (int i = 0; i < CS; ++i) acc[i] = 0.0f;
   const float2* ml2 = reinterpret_cast<const float2*>(a.part_ml);
-  // Up to R1 splits: one round of loads, the max taken from the loaded
-  // (m, l) pairs; more: a max pass, then the weighted sum.  Either way the
+  // Up to R1 splits: one round of loads (of two partials up to two splits, so
+  // that short contexts do not read one eight times), the max taken from the
+  // loaded (m, l) pairs; more: a max pass, then the weighted sum.  Either way the
   // splits are summed in ascending order with the same operands.
   constexpr int R1 = 8;
-  if (ns <= R1) {
-    float2 mlv[R1];
-    float4 ov[R1][CS / 4];
+  auto one_round = [&](auto rc) {
+    constexpr int R = decltype(rc)::value;
+    float2 mlv[R];
+    float4 ov[R][CS / 4];
 #pragma unroll
-    for (int q = 0; q < R1; ++q) {
+    for (int q = 0; q < R; ++q) {
       const size_t pi = (size_t)(base + min(q, ns - 1)) * a.ucols + col;
       mlv[q] = ml2[pi];
       const float4* po = reinterpret_cast<const float4*>(a.part_o + pi * a.hd + d0);
@@ -409,9 +413,9 @@ __global__ __launch_bounds__(NT) void combine_kernel(CombineArgs a) {
       for (int r = 0; r < CS / 4; ++r) ov[q][r] = po[r];
     }
 #pragma unroll
-    for (int q = 0; q < R1; ++q) mx = fmaxf(mx, mlv[q].x);
+    for (int q = 0; q < R; ++q) mx = fmaxf(mx, mlv[q].x);
 #pragma unroll
-    for (int q = 0; q < R1; ++q) {
+    for (int q = 0; q < R; ++q) {
       if (q >= ns || mlv[q].x == -INFINITY) continue;
       const float f = exp2f(mlv[q].x - mx);
       L += f * mlv[q].y;
@@ -423,7 +427,9 @@ __global__ __launch_bounds__(NT) void combine_kernel(CombineArgs a) {
         acc[4 * r + 3] += f * ov[q][r].w;
       }
     }
-  }
+  };
+  if (ns <= 2) one_round(std::integral_constant<int, 2>{});
+  else if (ns <= R1) one_round(std::integral_constant<int, R1>{});
   for (int s0 = 0; s0 < (ns <= R1 ? 0 : ns); s0 += 4) {
     float mm[4];
 #pragma unroll
