@@ -221,7 +221,7 @@ hipError_t launch_lmhead(LmHeadArgs& a, hipStream_t st) {
   a.nparts = lmhead_nparts(a.V);
   LmP p{a.a, a.as, a.wcodes, a.wscale, a.logits, a.part_val, a.part_idx, a.W, a.V, a.H, a.H / 64};
   hipError_t e;
-  // Four steps in flight take 157 VGPRs: three waves a SIMD, 3072 on the chip,
+  // Four steps in flight take 164 VGPRs: three waves a SIMD, 3072 on the chip,
   // where one step holds four.  A round of three costs about 0.7 of one of
   // four (0.8 at 16 K steps and fewer), so the whole rounds decide (us with the
   // reduce, four steps / one: H 1024, V 32000, 192 rows' 3000 waves 37.8 / 40.9,
