@@ -395,10 +395,12 @@ __global__ __launch_bounds__(NT) void combine_kernel(CombineArgs a) {
 #pragma unroll
   for (int i = 0; i < CS; ++i) acc[i] = 0.0f;
   const float2* ml2 = reinterpret_cast<const float2*>(a.part_ml);
-  // Up to R1 splits: one round of loads (of two partials up to two splits, so
-  // that short contexts do not read one eight times), the max taken from the
-  // loaded (m, l) pairs; more: a max pass, then the weighted sum.  Either way the
-  // splits are summed in ascending order with the same operands.
+  // Up to R1 splits: one round of loads, the max taken from the loaded (m, l)
+  // pairs; more: a max pass, then the weighted sum.  Either way the splits are
+  // summed in ascending order with the same operands.  Up to two splits a wide
+  // row loads two partials and not one of them eight times (32 heads, 513 rows
+  // of one split 11.8 -> 10.2 us; at 256 threads the branch costs 0.3 and gives
+  // nothing).
   constexpr int R1 = 8;
   auto one_round = [&](auto rc) {
     constexpr int R = decltype(rc)::value;
@@ -428,7 +430,7 @@ __global__ __launch_bounds__(NT) void combine_kernel(CombineArgs a) {
       }
     }
   };
-  if (ns <= 2) one_round(std::integral_constant<int, 2>{});
+  if (NT > 256 && ns <= 2) one_round(std::integral_constant<int, 2>{});
   else if (ns <= R1) one_round(std::integral_constant<int, R1>{});
   for (int s0 = 0; s0 < (ns <= R1 ? 0 : ns); s0 += 4) {
     float mm[4];
